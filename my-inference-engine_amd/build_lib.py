@@ -1,9 +1,10 @@
-"""Build libmi_fa2.so (the HIP kernels + C ABI) in-tree with hipcc for gfx950.
+"""Build libmi_fa2.so and libmi_model.so (the HIP kernels + C ABIs) in-tree with hipcc for gfx950.
 
     python my-inference-engine_amd/build_lib.py
 
-Compiles every source of csrc/ in parallel into _build/ and links kernels/libmi_fa2.so, which
-kernels/_lib.py loads.  Always rebuilds (a few seconds per file).
+Compiles every source of csrc/ in parallel into _build/ and links kernels/libmi_fa2.so (attention,
+sampling, step metadata; loaded by kernels/_lib.py) and kernels/libmi_model.so (the projections of
+few rows; loaded by kernels/few_rows.py).  Always rebuilds (a few seconds per file).
 """
 import os
 import subprocess
@@ -16,7 +17,11 @@ ROOT = PKG.parent
 CSRC = PKG / "csrc"
 BUILD = PKG / "_build"
 OUT = PKG / "kernels" / "libmi_fa2.so"
-SOURCES = ["fa2_prefill.hip", "fa2_decode.hip", "fa2_general.hip", "fa2_merge.hip", "rope_kv.hip", "sample.hip", "step_meta.hip", "model_ops.hip", "fa2_capi.cpp"]
+LIBS = {
+    OUT: ["fa2_prefill.hip", "fa2_decode.hip", "fa2_general.hip", "fa2_merge.hip", "rope_kv.hip",
+          "sample.hip", "step_meta.hip", "model_ops.hip", "fa2_capi.cpp"],
+    PKG / "kernels" / "libmi_model.so": ["linear_rows.hip", "model_capi.cpp"],
+}
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 ARCH = "gfx950"
@@ -47,16 +52,19 @@ def _compile(src: str) -> Path:
 
 def build(verbose: bool = True) -> Path:
     BUILD.mkdir(exist_ok=True)
-    with ThreadPoolExecutor(max_workers=len(SOURCES)) as ex:
-        objs = list(ex.map(_compile, SOURCES))
-    tmp = OUT.with_suffix(".so.tmp")
-    cmd = [HIPCC, f"--offload-arch={ARCH}", "-shared", "-fPIC", *map(str, objs), "-o", str(tmp)]
-    proc = subprocess.run(cmd, capture_output=True, text=True)
-    if proc.returncode != 0:
-        raise RuntimeError(f"link failed:\n{' '.join(cmd)}\n{proc.stdout}{proc.stderr}")
-    os.replace(tmp, OUT)
-    if verbose:
-        print(f"built {OUT.relative_to(ROOT)}")
+    sources = [src for srcs in LIBS.values() for src in srcs]
+    with ThreadPoolExecutor(max_workers=len(sources)) as ex:
+        objs = dict(zip(sources, ex.map(_compile, sources)))
+    for out, srcs in LIBS.items():
+        tmp = out.with_suffix(".so.tmp")
+        cmd = [HIPCC, f"--offload-arch={ARCH}", "-shared", "-fPIC", *(str(objs[x]) for x in srcs),
+               "-o", str(tmp)]
+        proc = subprocess.run(cmd, capture_output=True, text=True)
+        if proc.returncode != 0:
+            raise RuntimeError(f"link failed:\n{' '.join(cmd)}\n{proc.stdout}{proc.stderr}")
+        os.replace(tmp, out)
+        if verbose:
+            print(f"built {out.relative_to(ROOT)}")
     return OUT
 
 

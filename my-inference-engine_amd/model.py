@@ -14,10 +14,13 @@ logits (model.py:204-207) -- with two deliberate differences on the GPU path:
   * Each residual add and the RMSNorm after it are one HIP launch (kernels.model_ops.add_rmsnorm)
     and SiLU x up is one more (kernels.model_ops.silu_mul), instead of about twenty small torch
     launches per layer, with the same rounding points.
-  * The gate/up GEMM and the tied lm_head multiply by a cached transposed copy of their weight
-    ([in, out] row-major): at decode sizes hipBLASLt picks much faster kernels for that layout of
-    these two shapes (the other projections are faster as they are).  The parameters keep the
-    reference's layout; the copy is rebuilt if a weight changes.
+  * A step of few tokens (a decode step's rows) runs its projections on hand-written kernels
+    (kernels.few_rows) that stream the weights in their own layout and do the norm, RoPE and cache
+    write, SwiGLU and residual add of each in the same launch: four launches per layer beside
+    attention's, with the same rounding points.
+  * For more tokens the gate/up GEMM and the tied lm_head multiply by a cached transposed copy of
+    their weight ([in, out] row-major), the layout hipBLASLt has the faster kernels for.  The
+    parameters keep the reference's layout; the copy is rebuilt if a weight changes.
 
 forward_mixed() runs one step over rows that append different numbers of tokens -- decoding chats
 (one token each) and newly admitted prompts -- packed back to back: every projection, norm and MLP
@@ -36,6 +39,7 @@ import torch
 import torch.nn as nn
 import torch.nn.functional as F
 
+from kernels import few_rows
 from kernels.fa2 import fa2_paged, fa2_paged_varlen
 from kernels.model_ops import add_rmsnorm, silu_mul
 from kernels.rope import rope_kv_write
@@ -93,6 +97,21 @@ def transposed(weight):
     return cached[1]
 
 
+def plain(*modules):
+    """Whether the modules are exactly these classes with nothing hooked on, so that a kernel may do
+    their work without calling them."""
+    return (not nn.modules.module._has_any_global_hook()
+            and all(type(m) in (nn.Linear, RMSNorm, Attention, MLP, Block)
+                    and not (m._forward_hooks or m._forward_pre_hooks or m._backward_hooks
+                             or m._backward_pre_hooks) for m in modules))
+
+
+def inference(*tensors):
+    """Whether nothing would record a gradient or cast the inputs: the fused kernels do neither."""
+    return (not (torch.is_grad_enabled() and any(t.requires_grad for t in tensors))
+            and not torch.is_autocast_enabled("cuda"))
+
+
 def repeat_kv(x, n_rep):
     if n_rep == 1:
         return x
@@ -139,14 +158,7 @@ class Attention(nn.Module):
                               sin[:, 0].reshape(B * T, cfg.head_dim), meta.slot_mapping32,
                               cache.k_pool(layer), cache.v_pool(layer), cfg.num_heads,
                               cfg.num_kv_heads)
-            if meta.packed:
-                out = self._attend_packed(q.view(B * T, cfg.num_heads, cfg.head_dim), cache,
-                                          layer, meta)
-                return self.o_proj(out.view(B, T, self.q_size))
-            q = q.view(B, T, cfg.num_heads, cfg.head_dim).transpose(1, 2)
-            out = fa2_paged(q, cache.k_pool(layer), cache.v_pool(layer), meta.block_table,
-                            meta.kv_lens, block_size=cache.block_size, max_kv_len=meta.max_kv,
-                            is_causal=T > 1)
+            return self.o_proj(self._attend(q, B, T, cache, layer, meta))
         else:
             q, k, v = qkv.split([self.q_size, self.kv_size, self.kv_size], dim=-1)
             q = q.view(B, T, cfg.num_heads, cfg.head_dim).transpose(1, 2)
@@ -160,6 +172,38 @@ class Attention(nn.Module):
             k_all, v_all = cache.read(layer, meta)
             out = sdpa_fallback(q, k_all, v_all, meta.starts, cfg.num_heads // cfg.num_kv_heads)
         return self.o_proj(out.transpose(1, 2).reshape(B, T, self.q_size))
+
+    def _attend(self, q, B, T, cache, layer, meta):
+        """Attention of the rotated queries q [B * T, Hq * d] over the cache -> [B, T, Hq * d]."""
+        cfg = self.cfg
+        if meta.packed:
+            out = self._attend_packed(q.view(B * T, cfg.num_heads, cfg.head_dim), cache, layer, meta)
+            return out.view(B, T, self.q_size)
+        q = q.view(B, T, cfg.num_heads, cfg.head_dim).transpose(1, 2)
+        out = fa2_paged(q, cache.k_pool(layer), cache.v_pool(layer), meta.block_table,
+                        meta.kv_lens, block_size=cache.block_size, max_kv_len=meta.max_kv,
+                        is_causal=T > 1)
+        return out.transpose(1, 2).reshape(B, T, self.q_size)
+
+    def few_rows_fit(self, x, norm):
+        """Whether few_rows_step takes x [tokens, hidden]."""
+        qkv, o = self.qkv_proj, self.o_proj
+        return (plain(self, norm, qkv, o) and self.cfg.head_dim == few_rows.HEAD_DIM
+                and few_rows.linear_fits(x, qkv.weight, norm.weight)
+                and qkv.weight.shape[0] == self.q_size + 2 * self.kv_size
+                and few_rows.weight_fits(o.weight, x, x.shape[1])
+                and o.weight.shape[1] == self.q_size and o.bias is None)
+
+    def few_rows_step(self, res, norm, shape, cos, sin, cache, layer, meta):
+        """res [tokens, hidden] += attention of norm(res), in three launches and attention's own."""
+        cfg = self.cfg
+        (B, T, _), n = shape, res.shape[0]
+        q = few_rows.qkv_rope(res, norm.weight, cfg.rms_norm_eps, self.qkv_proj.weight, self.qkv_proj.bias,
+                              cos[:, 0].reshape(n, cfg.head_dim), sin[:, 0].reshape(n, cfg.head_dim),
+                              meta.slot_mapping32, cache.k_pool(layer), cache.v_pool(layer),
+                              cfg.num_heads, cfg.num_kv_heads)
+        a = self._attend(q, B, T, cache, layer, meta).view(n, self.q_size)
+        few_rows.linear(a, self.o_proj.weight, residual=res, out=res)
 
     def _attend_packed(self, q, cache, layer, meta):
         """q [N, Hq, d] packed queries of a mixed step -> [N, Hq, d]: the leading one-token rows
@@ -202,12 +246,24 @@ class MLP(nn.Module):
 
     def forward(self, x):
         if x.is_cuda:
-            gu = x.reshape(-1, x.shape[-1]) @ transposed(self.gate_up_proj.weight)
+            rows = x.reshape(-1, x.shape[-1])
+            if rows.shape[0] <= few_rows.MAX_ROWS and self.few_rows_fit(rows):
+                return few_rows.mlp(rows, self.gate_up_proj.weight,
+                                    self.down_proj.weight).view(x.shape)
+            gu = rows @ transposed(self.gate_up_proj.weight)
             act = silu_mul(gu).view(*x.shape[:-1], self.inter)
             return self.down_proj(act)
         gu = self.gate_up_proj(x)
         gate, up = gu.split(self.inter, dim=-1)
         return self.down_proj(F.silu(gate) * up)
+
+    def few_rows_fit(self, x, norm=None):
+        """Whether few_rows.mlp does this module's work on x [tokens, hidden] (after `norm`)."""
+        gu, down = self.gate_up_proj, self.down_proj
+        return (plain(gu, down, *((self, norm) if norm is not None else ()))
+                and gu.bias is None and down.bias is None and inference(x, gu.weight, down.weight)
+                and few_rows.mlp_fits(x, gu.weight, down.weight,
+                                      norm.weight if norm is not None else None))
 
 
 class Block(nn.Module):
@@ -273,9 +329,14 @@ class Qwen2ForCausalLM(nn.Module):
 
     def lm_head(self, x):
         """Tied-embedding logits (model.py:204-207)."""
+        w = self.embed_tokens.weight
         if x.is_cuda:
-            return x @ transposed(self.embed_tokens.weight)
-        return x @ self.embed_tokens.weight.T
+            rows = x.reshape(-1, x.shape[-1])
+            if (rows.shape[0] <= few_rows.MAX_ROWS and inference(x, w)
+                    and few_rows.linear_fits(rows, w)):
+                return few_rows.linear(rows, w).view(*x.shape[:-1], w.shape[0])
+            return x @ transposed(w)
+        return x @ w.T
 
     def run_layers(self, x, cos, sin, cache, meta):
         """The decoder layers over x [B, T, hidden].  On the GPU each residual add is fused with the
@@ -287,6 +348,14 @@ class Qwen2ForCausalLM(nn.Module):
             return x
         shape, H, eps = x.shape, x.shape[-1], self.cfg.rms_norm_eps
         res = x.reshape(-1, H)
+        if self._few_rows_fit(res):
+            for i, layer in enumerate(self.layers):
+                layer.self_attn.few_rows_step(res, layer.input_layernorm, shape, cos, sin, cache, i,
+                                              meta)
+                norm, mlp = layer.post_attention_layernorm, layer.mlp
+                few_rows.mlp(res, mlp.gate_up_proj.weight, mlp.down_proj.weight, residual=res,
+                             norm_weight=norm.weight, eps=eps, out=res)
+            return res.view(shape)
         _, h = add_rmsnorm(res, self.layers[0].input_layernorm.weight, eps)
         for i, layer in enumerate(self.layers):
             a = layer.self_attn(h.view(shape), cos, sin, cache, i, meta).reshape(-1, H)
@@ -299,6 +368,13 @@ class Qwen2ForCausalLM(nn.Module):
             else:
                 res = res + m
         return res.view(shape)
+
+    def _few_rows_fit(self, res):
+        """Whether every layer of a step over res [tokens, hidden] runs on the few-row kernels."""
+        return (1 <= res.shape[0] <= few_rows.MAX_NORM_ROWS and inference(res, *self.parameters())
+                and all(layer.self_attn.few_rows_fit(res, layer.input_layernorm)
+                        and layer.mlp.few_rows_fit(res, layer.post_attention_layernorm)
+                        for layer in self.layers))
 
     def forward_mixed(self, rows, cache, seqs):
         """One packed step: rows[b] (a list of token ids, at least one) is appended to cache
