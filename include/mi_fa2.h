@@ -113,7 +113,9 @@ MI_FA2_API int mi_fa2_set_clock_probe(uint64_t* probe);
  *   row uses all seqlen_k keys, kernels/fa2.py:182-183; values are clamped to [0, seqlen_k]).
  *   q_strides/k_strides/v_strides/o_strides: 4 strides each; lse_strides: 3 (ignored if lse NULL).
  * seqlen_q == 1 runs the split-KV decode kernel, which needs the workspace; seqlen_q > 1 runs the
- * MFMA prefill kernel, which needs none.
+ * MFMA prefill kernel, which needs none.  Where few queries meet many keys, a non-zero size is
+ * reported for seqlen_q > 1 too: with that workspace (16-byte aligned) the keys are split over
+ * work-groups, without it the call runs unsplit.
  */
 MI_FA2_API size_t mi_fa2_fwd_workspace_size(int32_t batch, int32_t heads_q, int32_t heads_kv,
                                  int32_t seqlen_q, int32_t seqlen_k, int32_t head_dim);

@@ -16,6 +16,11 @@
 namespace mi_fa2 {
 hipError_t launch_prefill(const FwdParams& p, int dtype, int mode, int max_seqlen_q,
                           hipStream_t stream);
+int prefill_split_pieces(int n_cus, int64_t batch, int heads_q, int heads_kv, int64_t seqlen_q,
+                         int64_t max_kv);
+size_t prefill_split_bytes(int64_t batch, int heads_q, int heads_kv, int64_t seqlen_q, int pieces);
+hipError_t launch_prefill_split(const FwdParams& p, int dtype, int mode, int pieces,
+                                hipStream_t stream);
 hipError_t launch_decode(const FwdParams& p, int dtype, int mode, hipStream_t stream);
 hipError_t launch_general(const FwdParams& p, int dtype, int d, int dv, hipStream_t stream);
 hipError_t launch_merge(const MergeParams& p, int out_dtype, hipStream_t stream);
@@ -174,6 +179,31 @@ size_t decode_workspace(int64_t batch, int64_t heads_q, int64_t heads_kv, int64_
   if (splits <= 1) return 0;
   return (size_t)batch * heads_q * splits * (mi_fa2::kHeadDim + 2) * sizeof(float) +
          (size_t)batch * heads_kv * sizeof(int32_t);
+}
+
+// The padded prefill's workspace, where cutting the tiles' keys into pieces pays: sized for the CUs
+// of a whole MI355X (a launch on a device with fewer cuts into fewer pieces).  It is optional: a
+// call without it runs unsplit.
+constexpr int kSplitCus = 256;
+size_t split_workspace(int64_t batch, int heads_q, int heads_kv, int64_t seqlen_q, int64_t max_kv) {
+  const int pieces =
+      mi_fa2::prefill_split_pieces(kSplitCus, batch, heads_q, heads_kv, seqlen_q, max_kv);
+  return mi_fa2::prefill_split_bytes(batch, heads_q, heads_kv, seqlen_q, pieces);
+}
+
+int launched(hipError_t err);
+
+// The padded prefill of p, split if the workspace allows.
+int run_prefill(FwdParams& p, const Plan& plan, int dtype, int mode, void* workspace,
+                size_t workspace_bytes, hipStream_t s) {
+  const int pieces = mi_fa2::prefill_split_pieces(std::min(plan.cus, kSplitCus), p.B, p.Hq, p.Hkv,
+                                                  p.T, p.S);
+  const size_t need = mi_fa2::prefill_split_bytes(p.B, p.Hq, p.Hkv, p.T, pieces);
+  if (need && workspace && workspace_bytes >= need && aligned16(workspace)) {
+    p.ws_o = static_cast<float*>(workspace);
+    return launched(mi_fa2::launch_prefill_split(p, dtype, mode, pieces, s));
+  }
+  return launched(mi_fa2::launch_prefill(p, dtype, mode, p.T, s));
 }
 
 void set_workspace(FwdParams& p, void* workspace) {
@@ -350,7 +380,7 @@ int fwd_paged(int32_t dtype, const void* q, const void* k_pool, const void* v_po
   }
   if (int rc = check_prefill_strides(p.k_st, p.v_st)) return rc;
   if (int rc = set_device(p, &plan)) return rc;
-  return launched(mi_fa2::launch_prefill(p, dtype, mi_fa2::kPaged, seqlen_q, s));
+  return run_prefill(p, plan, dtype, mi_fa2::kPaged, workspace, workspace_bytes, s);
 }
 
 }  // namespace
@@ -389,8 +419,11 @@ int mi_fa2_set_clock_probe(uint64_t* probe) {
 size_t mi_fa2_fwd_workspace_size(int32_t batch, int32_t heads_q, int32_t heads_kv,
                                  int32_t seqlen_q, int32_t seqlen_k, int32_t head_dim) {
   (void)head_dim;
-  if (heads_kv <= 0 || heads_q % heads_kv || !uses_decode(seqlen_q, heads_q / heads_kv, batch))
+  if (batch <= 0 || heads_q <= 0 || heads_kv <= 0 || heads_q % heads_kv || seqlen_q <= 0 ||
+      seqlen_k <= 0)
     return 0;
+  if (!uses_decode(seqlen_q, heads_q / heads_kv, batch))
+    return split_workspace(batch, heads_q, heads_kv, seqlen_q, seqlen_k);
   return decode_workspace(batch, heads_q, heads_kv, seqlen_k);
 }
 
@@ -455,7 +488,7 @@ int mi_fa2_fwd(int32_t dtype, const void* q, const void* k, const void* v, void*
   }
   if (int rc = check_prefill_strides(p.k_st, p.v_st)) return rc;
   if (int rc = set_device(p, &plan)) return rc;
-  return launched(mi_fa2::launch_prefill(p, dtype, mi_fa2::kDense, seqlen_q, s));
+  return run_prefill(p, plan, dtype, mi_fa2::kDense, workspace, workspace_bytes, s);
 }
 
 int mi_fa2_fwd_general(int32_t dtype, const void* q, const void* k, const void* v, void* o,

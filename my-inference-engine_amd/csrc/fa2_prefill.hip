@@ -103,25 +103,6 @@ inline int prefill_grid_size(int classes, int group, int n_qt, int xcd_log2) {
   return X * ((stride * n_qt + X - 1) / X) * group;
 }
 
-// Division by a divisor fixed for the launch, as a multiply: n / d = umulhi(n, m) >> l with
-// l = floor(log2 d) and m = floor(2^(32+l) / d) + 1, exact for n < 2^31 (the error term n*(m*d -
-// 2^(32+l)) / (d*2^(32+l)) < n / 2^(32+l) stays below 1/d); m = 0 marks a power of two (n >> l).
-// The work-group's item is found at its start, before any load can be issued, and the runtime
-// integer divisions this replaces cost a few hundred dependent instructions (1-3% on grids of many
-// short tiles).
-struct FastDiv {
-  uint32_t m, l, d;
-};
-inline FastDiv make_fastdiv(uint32_t d) {
-  FastDiv f{0, 0, d};
-  while ((2u << f.l) <= d && f.l < 31) ++f.l;
-  if ((d & (d - 1)) != 0) f.m = (uint32_t)(((uint64_t)1 << (32 + f.l)) / d + 1);
-  return f;
-}
-__device__ __forceinline__ int fdiv(int n, const FastDiv& f) {
-  return (int)(f.m ? __umulhi((uint32_t)n, f.m) >> f.l : (uint32_t)n >> f.l);
-}
-
 // The launch's item map: the divisors of prefill_item, log2 of the device's XCD count and, when
 // the classes divide the XCDs, log2 of the XCDs per class (else -1).
 struct ItemMap {
@@ -203,10 +184,49 @@ __device__ inline bool prefill_item_packed(const FwdParams& p, int w, const Item
   return r < n_qt;
 }
 
-template <typename E, int MODE, int NS>
+// Launches of few query tiles over many keys (a chat's next message over its cached history): one
+// work-group per query tile would leave most CUs idle and walk all the keys in one chain (150 new
+// queries over 3,001 keys: 24 work-groups of 24 steps, 42 us).  SP = true cuts each tile's keys
+// into `pieces` and packs the query heads of a kv head into shared tiles: row r of a tile is query
+// r / group of head r % group, so few queries still fill the 128 rows and a kv head's keys are read
+// by fewer tiles.  Each work-group leaves its rows' (O, m, l) in the workspace, in the accumulator
+// layout, and fa2_prefill_combine_kernel merges the pieces.
+//
+// Items are numbered (class, piece, tile), tile fastest: neighbours read the same keys.  XCD x runs
+// the x-th contiguous share of them, so the shares are even and one L2 serves a piece's tiles.
+struct SplitMap {
+  FastDiv tiles, pieces, hkv;
+  int32_t items, per_xcd, xcd_log2;
+};
+
+__device__ inline bool split_item(int w, const SplitMap& m, int& b, int& hk, int& piece, int& tile) {
+  const int item = (w & ((1 << m.xcd_log2) - 1)) * m.per_xcd + (w >> m.xcd_log2);
+  const int cp = fdiv(item, m.tiles);
+  tile = item - cp * (int)m.tiles.d;
+  const int c = fdiv(cp, m.pieces);
+  piece = cp - c * (int)m.pieces.d;
+  b = fdiv(c, m.hkv);
+  hk = c - b * (int)m.hkv.d;
+  return (w >> m.xcd_log2) < m.per_xcd && item < m.items;
+}
+
+// One work-group's partials: 128 rows of fp32 O in [wave][8][64 lanes] f32x4 order, then m and l.
+constexpr int kPartO = kPfRows * kHeadDim;
+constexpr int kPartFloats = kPartO + 2 * kPfRows;
+
+// Keys of piece `piece` of the tile whose last row is query q_last: whole blocks and steps.
+__device__ __forceinline__ void split_keys(int kv_hi, int unit, int piece, int pieces, int& k0,
+                                           int& k1) {
+  const int n = (kv_hi + unit - 1) / unit;
+  k0 = (int)((int64_t)piece * n / pieces) * unit;
+  k1 = min(kv_hi, (int)((int64_t)(piece + 1) * n / pieces) * unit);
+}
+
+template <typename E, int MODE, int NS, bool SP, typename Map>
 __global__ __launch_bounds__(PfShape<NS>::kThreads, 2) void fa2_prefill_kernel(const FwdParams p,
                                                                                int n_qt_max,
-                                                                               const ItemMap map) {
+                                                                               const Map map) {
+  static_assert(!SP || (NS == 2 && (MODE == kDense || MODE == kPaged)), "split launches");
   using Sh = PfShape<NS>;
   constexpr int kPfStep = Sh::kStep, kStageBytes = Sh::kStage, kVRegion = Sh::kVRegion;
   constexpr int kPfWaves = Sh::kWaves, kLpw = Sh::kLoadsPerWave;
@@ -218,9 +238,11 @@ __global__ __launch_bounds__(PfShape<NS>::kThreads, 2) void fa2_prefill_kernel(c
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int rg = wave % kPfRowGroups;
   const int ks = NS == 2 ? wave / kPfRowGroups : 0;  // key stream
-  int b, h, rank;
+  int b, h, rank, piece = 0;
   bool real;
-  if constexpr (MODE == kVarlen || MODE == kPagedVarlen)
+  if constexpr (SP)
+    real = split_item(blockIdx.x, map, b, h, piece, rank);  // h: the kv head, rank: the tile
+  else if constexpr (MODE == kVarlen || MODE == kPagedVarlen)
     real = p.B <= 64 ? prefill_item_packed(p, blockIdx.x, map, n_qt_max, b, h, rank)
                      : prefill_item(blockIdx.x, map, n_qt_max, b, h, rank);
   else
@@ -232,7 +254,14 @@ __global__ __launch_bounds__(PfShape<NS>::kThreads, 2) void fa2_prefill_kernel(c
   b = __builtin_amdgcn_readfirstlane(b);
   h = __builtin_amdgcn_readfirstlane(h);
   rank = __builtin_amdgcn_readfirstlane(rank);
-  const int hk = __builtin_amdgcn_readfirstlane(fdiv(h, map.group));
+  int hk;
+  if constexpr (SP) {
+    hk = h;
+    h = hk * p.group;
+    piece = __builtin_amdgcn_readfirstlane(piece);
+  } else {
+    hk = __builtin_amdgcn_readfirstlane(fdiv(h, map.group));
+  }
 
   int T_b, kv_len;
   int64_t q_off, o_off, l_off, k_off, v_off;
@@ -270,25 +299,48 @@ __global__ __launch_bounds__(PfShape<NS>::kThreads, 2) void fa2_prefill_kernel(c
   kv_len = __builtin_amdgcn_readfirstlane(kv_len);
   k_off = (int64_t)uniform_u64((uint64_t)k_off);
   v_off = (int64_t)uniform_u64((uint64_t)v_off);
-  const int n_qt = (T_b + kPfRows - 1) / kPfRows;
-  const int tile = n_qt - 1 - rank;
+  // Rows of the query tiles, and the query a row holds.
+  const int n_rows = SP ? T_b * p.group : T_b;
+  const FastDiv group_div = p.group_div;
+  const auto query_of = [&](int row) {
+    if constexpr (SP) return fdiv(row, group_div);
+    return row;
+  };
+  const int n_qt = (n_rows + kPfRows - 1) / kPfRows;
+  const int tile = SP ? rank : n_qt - 1 - rank;
   if (tile < 0) return;
   const int q0 = tile * kPfRows;
-  const int off = kv_len - T_b;  // query i sits at key position i + off
+  int off = kv_len - T_b;  // query i sits at key position i + off
 
   // Keys the work-group needs: up to what its last valid query row sees.
   int kv_hi = kv_len;
-  if (p.causal) kv_hi = min(kv_len, min(q0 + kPfRows, T_b) + off);
+  if (p.causal) kv_hi = min(kv_len, query_of(min(q0 + kPfRows, n_rows) - 1) + 1 + off);
   if (kv_hi < 0) kv_hi = 0;
+  int64_t bt_off = (int64_t)b * p.bt_stride;
+  if constexpr (SP) {
+    // This piece's keys, renumbered from 0.
+    int k0, k1;
+    split_keys(kv_hi, is_paged(MODE) ? max(kPfStep, p.block_size) : kPfStep, piece,
+               (int)map.pieces.d, k0, k1);
+    kv_hi = max(k1 - k0, 0);
+    kv_len = kv_hi;
+    off -= k0;
+    if constexpr (is_paged(MODE)) {
+      bt_off += k0 >> __builtin_ctz(p.block_size);
+    } else {
+      k_off += (int64_t)k0 * p.k_st;
+      v_off += (int64_t)k0 * p.v_st;
+    }
+  }
   kv_hi = __builtin_amdgcn_readfirstlane(kv_hi);  // uniform: keeps the load arithmetic scalar
   const int n_steps = (kv_hi + kPfStep - 1) / kPfStep;
 
   // This wave's rows and the key ranges they need.
   const int wq0 = q0 + rg * 32;
-  const bool wave_active = wq0 < T_b;
-  const int wq_last = min(wq0 + 31, T_b - 1);
+  const bool wave_active = wq0 < n_rows;
+  const int wq_last = query_of(min(wq0 + 31, n_rows - 1));
   const int wave_hi = p.causal ? min(kv_len, wq_last + off + 1) : kv_len;   // seen by some row
-  const int wave_full = p.causal ? min(kv_len, wq0 + off + 1) : kv_len;     // seen by every row
+  const int wave_full = p.causal ? min(kv_len, query_of(wq0) + off + 1) : kv_len;  // by every row
 
   const int r32 = lane & 31;
   const int g = lane >> 5;
@@ -297,8 +349,10 @@ __global__ __launch_bounds__(PfShape<NS>::kThreads, 2) void fa2_prefill_kernel(c
 
   // Q^T as the B operand: k-step s covers d = s*16 + g*8 + [0, 8).
   u32x4 qb[8];
-  if (qrow < T_b) {
-    const uint16_t* qp = p.q + q_off + (int64_t)qrow * p.q_st + g * 8;
+  const int qi = query_of(qrow);
+  if (qrow < n_rows) {
+    const uint16_t* qp = p.q + q_off + (int64_t)qi * p.q_st + g * 8;
+    if constexpr (SP) qp += (int64_t)(qrow - qi * p.group) * p.q_sh;
 #pragma unroll
     for (int s = 0; s < 8; ++s) qb[s] = ld16(qp + s * 16);
   } else {
@@ -311,7 +365,7 @@ __global__ __launch_bounds__(PfShape<NS>::kThreads, 2) void fa2_prefill_kernel(c
   for (int i = 0; i < 4; ++i) oacc[i] = f32x16{};
   float m_run = -INFINITY;  // running max of c*score (log2 units); -inf until a key is seen
   float l_run = 0.f;        // this lane's partial sum of exp2(c*score - m_run)
-  const int lim = p.causal ? min(kv_len, qrow + off + 1) : kv_len;  // keys < lim are visible
+  const int lim = p.causal ? min(kv_len, qi + off + 1) : kv_len;  // keys < lim are visible
 
   // Software pipeline.  Tile (j, s) is keys 128j + 64s .. +63.  Stream 0 (waves 0-3) works one
   // tile ahead of stream 1 (waves 4-7) in the score phase, so that in every step one wave of each
@@ -393,7 +447,7 @@ __global__ __launch_bounds__(PfShape<NS>::kThreads, 2) void fa2_prefill_kernel(c
       const int ts = t == 0 ? k0_start(j) : t == 1 ? k1_start(j) : t == 2 ? v0_start(j) : v1_start(j);
       const int r0 = ts + 4 * kLpw * wave;
       if (ts >= 0 && ts < kv_hi && r0 < kv_hi)
-        return p.block_table[(int64_t)b * p.bt_stride + (r0 >> __builtin_ctz(p.block_size))];
+        return p.block_table[bt_off + (r0 >> __builtin_ctz(p.block_size))];
       return -1;
     } else {
       return 0;
@@ -813,6 +867,26 @@ __global__ __launch_bounds__(PfShape<NS>::kThreads, 2) void fa2_prefill_kernel(c
     }
 
     const float l_tot = l_run + __shfl_xor(l_run, 32);
+    if constexpr (SP) {
+      // The rows' state goes to the workspace as it is: whole contiguous stores.
+      const int item = ((b * p.Hkv + hk) * (int)map.pieces.d + piece) * n_qt + tile;
+      float* part = p.ws_o + (int64_t)item * kPartFloats;
+      f32x4* po = reinterpret_cast<f32x4*>(part) + (rg * NS + ks) * 8 * 64 + lane;
+      if (wave_active) {   // the combine does not read row groups past the last row
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+          for (int rr = 0; rr < 4; ++rr)
+            po[(4 * i + rr) * 64] = f32x4{ok[i][rr * 4], ok[i][rr * 4 + 1], ok[i][rr * 4 + 2],
+                                          ok[i][rr * 4 + 3]};
+      }
+      if (ks == 0 && g == 0 && wave_active) {
+        part[kPartO + 32 * rg + r32] = m_run;
+        part[kPartO + kPfRows + 32 * rg + r32] = l_tot;
+      }
+      probe_mark(p.clock_probe, blockIdx.x, true);
+      return;
+    }
     const float inv = l_tot > 0.f ? 1.f / l_tot : 0.f;
     // Accumulator r of d-block db is d = 32*db + 8*(r/4) + 4*g + r%4: four consecutive d per group.
     // The wave's half rows go through LDS so that every global store writes whole 128-byte
@@ -848,6 +922,163 @@ __global__ __launch_bounds__(PfShape<NS>::kThreads, 2) void fa2_prefill_kernel(c
   probe_mark(p.clock_probe, blockIdx.x, true);
 }
 
+// Merges the pieces of a split launch's tiles and stores the rows.  One work-group per (tile, row
+// group, 32 dims); its four waves take a quarter of the pieces each and meet in LDS.  The lanes keep
+// the accumulator layout the pieces were written in, so a piece is four contiguous 1 KB reads.
+template <typename E>
+__global__ __launch_bounds__(256) void fa2_prefill_combine_kernel(const FwdParams p, int n_qt,
+                                                                  int pieces) {
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int db = blockIdx.x & 3, rg = (blockIdx.x >> 2) & 3, item = blockIdx.x >> 4;
+  const int c = item / n_qt, tile = item - c * n_qt;
+  const int n_rows = p.T * p.group;
+  if (tile * kPfRows + rg * 32 >= n_rows) return;
+  const int b = c / p.Hkv, hk = c - b * p.Hkv;
+  const int r32 = lane & 31, g = lane >> 5;
+  const int row = tile * kPfRows + rg * 32 + r32;
+  // piece s of the tile: item (class, s, tile)
+  const float* part = p.ws_o + ((int64_t)c * pieces * n_qt + tile) * kPartFloats;
+  const int64_t stride = (int64_t)n_qt * kPartFloats;
+  // wave (rg, ks = db / 2) wrote block i = db % 2 of its half
+  const int o_at = (((rg * 2 + (db >> 1)) * 8 + 4 * (db & 1)) * 64 + lane) * 4;
+  const int m_at = kPartO + 32 * rg + r32;
+  const int s_lo = wave * pieces / 4, s_hi = (wave + 1) * pieces / 4;
+  float M = -INFINITY, L = 0.f;
+  f32x4 acc[4];
+#pragma unroll
+  for (int k = 0; k < 4; ++k) acc[k] = f32x4{0.f, 0.f, 0.f, 0.f};
+  constexpr int kBatch = 4;   // pieces whose loads are in flight together
+  for (int s0 = s_lo; s0 < s_hi; s0 += kBatch) {
+    float m[kBatch], l[kBatch];
+    f32x4 o[kBatch][4];
+#pragma unroll
+    for (int u = 0; u < kBatch; ++u) {
+      const float* q = part + min(s0 + u, s_hi - 1) * stride;
+      m[u] = s0 + u < s_hi ? q[m_at] : -INFINITY;
+      l[u] = q[m_at + kPfRows];
+#pragma unroll
+      for (int k = 0; k < 4; ++k) o[u][k] = *reinterpret_cast<const f32x4*>(q + o_at + k * 256);
+    }
+    float Mn = M;
+#pragma unroll
+    for (int u = 0; u < kBatch; ++u) Mn = fmaxf(Mn, m[u]);
+    const float Mu = Mn == -INFINITY ? 0.f : Mn;
+    const float sc = exp2_fast(M - Mu);
+    L *= sc;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) acc[k] *= sc;
+#pragma unroll
+    for (int u = 0; u < kBatch; ++u) {
+      const float f = exp2_fast(m[u] - Mu);   // 0 for a piece none of whose keys the row sees
+      L = __builtin_fmaf(l[u], f, L);
+#pragma unroll
+      for (int k = 0; k < 4; ++k)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) acc[k][e] = __builtin_fmaf(o[u][k][e], f, acc[k][e]);
+    }
+    M = Mn;
+  }
+  __shared__ f32x4 so[4][4][64];
+  __shared__ float sm[4][64], sl[4][64];
+#pragma unroll
+  for (int k = 0; k < 4; ++k) so[wave][k][lane] = acc[k];
+  sm[wave][lane] = M;
+  sl[wave][lane] = L;
+  __syncthreads();
+  // wave k finishes dims 8k + 4g .. +3 of the block
+  float Mw[4], f[4];
+  M = -INFINITY;
+#pragma unroll
+  for (int u = 0; u < 4; ++u) M = fmaxf(M, Mw[u] = sm[u][lane]);
+  const float Mu = M == -INFINITY ? 0.f : M;
+  L = 0.f;
+  f32x4 o = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int u = 0; u < 4; ++u) {
+    f[u] = exp2_fast(Mw[u] - Mu);
+    L = __builtin_fmaf(sl[u][lane], f[u], L);
+    const f32x4 t = so[u][wave][lane];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) o[e] = __builtin_fmaf(t[e], f[u], o[e]);
+  }
+  if (row >= n_rows) return;
+  const int qi = fdiv(row, p.group_div), h = hk * p.group + row - qi * p.group;
+  const float inv = L > 0.f ? 1.f / L : 0.f;
+  uint16_t* op = p.o + (int64_t)b * p.o_sb + (int64_t)h * p.o_sh + (int64_t)qi * p.o_st;
+  *reinterpret_cast<u32x2*>(op + 32 * db + 8 * wave + 4 * g) =
+      u32x2{E::pack2(o[0] * inv, o[1] * inv), E::pack2(o[2] * inv, o[3] * inv)};
+  if (p.lse && db == 0 && wave == 0 && g == 0)
+    p.lse[(int64_t)b * p.l_sb + (int64_t)h * p.l_sh + (int64_t)qi * p.l_st] =
+        L > 0.f ? (M + __builtin_log2f(L)) * kLn2 : -INFINITY;
+}
+
+static int64_t split_tiles(int64_t batch, int heads_q, int heads_kv, int64_t seqlen_q) {
+  return batch * heads_kv * ((seqlen_q * (heads_q / heads_kv) + kPfRows - 1) / kPfRows);
+}
+
+// Pieces each tile's keys are cut into for a padded launch (1: none) on a device of n_cus CUs, the
+// number with the least time by this model (us, fitted to 18 shapes of 5 to 700 queries over 900 to
+// 8,000 keys at 1 to 63 pieces, within 10% of the best of them everywhere):
+//   unsplit, one work-group per CU or fewer:  6.5 + 1.45 per 128-key step of the longest tile;
+//   split, one work-group per CU or fewer:    9.5 + 1.45 per step of a piece
+//       + 0.033 per tile and piece (its partials written and read) + 0.05 per piece (the merge).
+// Measured unsplit -> split: 150 queries over 3,001 keys 42.4 -> 19.6 us, 5 over 8,000 92.6 -> 13.9,
+// 700 over 4,000 53.9 -> 35.8; 700 over 1,000 stays unsplit (19.1, split 21.8).
+int prefill_split_pieces(int n_cus, int64_t batch, int heads_q, int heads_kv, int64_t seqlen_q,
+                         int64_t max_kv) {
+  const int64_t unsplit = batch * heads_q * ((seqlen_q + kPfRows - 1) / kPfRows);
+  if (seqlen_q < 1 || unsplit < 1 || unsplit > n_cus) return 1;
+  const int64_t tiles = split_tiles(batch, heads_q, heads_kv, seqlen_q);
+  const int64_t row_groups =   // of 32 rows, four to a tile: what is written
+      batch * heads_kv * ((seqlen_q * (heads_q / heads_kv) + 31) / 32);
+  const int64_t steps = (max_kv + PfShape<2>::kStep - 1) / PfShape<2>::kStep;
+  const int64_t most = std::min<int64_t>(n_cus / tiles, steps);
+  int best = 1;
+  int64_t best_cost = 650 + 145 * steps - 100;   // in 10 ns; a split has to gain 1 us
+  for (int64_t s = 2; s <= most; ++s) {
+    const int64_t each = (steps + s - 1) / s;
+    const int64_t cost = 950 + 145 * each + 33 * row_groups * s / 40 + 5 * s;
+    if (cost < best_cost) {
+      best_cost = cost;
+      best = (int)s;
+    }
+  }
+  return best;
+}
+
+size_t prefill_split_bytes(int64_t batch, int heads_q, int heads_kv, int64_t seqlen_q, int pieces) {
+  return pieces > 1 ? (size_t)split_tiles(batch, heads_q, heads_kv, seqlen_q) * pieces *
+                          kPartFloats * sizeof(float)
+                    : 0;
+}
+
+// The split launch of p (padded modes): p.ws_o holds prefill_split_bytes.
+template <typename E, int MODE>
+static hipError_t launch_prefill_split_t(FwdParams p, int pieces, hipStream_t stream) {
+  const int n_qt = (int)(((int64_t)p.T * p.group + kPfRows - 1) / kPfRows);
+  const int items = p.B * p.Hkv * pieces * n_qt, X = 1 << p.xcd_log2;
+  p.group_div = make_fastdiv(p.group);
+  const SplitMap map{make_fastdiv(n_qt), make_fastdiv(pieces), make_fastdiv(p.Hkv), items,
+                     (items + X - 1) / X, p.xcd_log2};
+  hipLaunchKernelGGL((fa2_prefill_kernel<E, MODE, 2, true, SplitMap>), dim3(map.per_xcd * X),
+                     dim3(PfShape<2>::kThreads), 0, stream, p, n_qt, map);
+  hipError_t err = hipGetLastError();
+  if (err != hipSuccess) return err;
+  hipLaunchKernelGGL((fa2_prefill_combine_kernel<E>), dim3(p.B * p.Hkv * n_qt * 16), dim3(256), 0,
+                     stream, p, n_qt, pieces);
+  return hipGetLastError();
+}
+
+hipError_t launch_prefill_split(const FwdParams& p, int dtype, int mode, int pieces,
+                                hipStream_t stream) {
+  if (dtype == 0)
+    return mode == kPaged ? launch_prefill_split_t<BF16, kPaged>(p, pieces, stream)
+                          : launch_prefill_split_t<BF16, kDense>(p, pieces, stream);
+  return mode == kPaged ? launch_prefill_split_t<FP16, kPaged>(p, pieces, stream)
+                        : launch_prefill_split_t<FP16, kDense>(p, pieces, stream);
+}
+
 // Key streams per work-group for a launch of `grid` work-groups whose query tiles see at most
 // `max_keys` keys.  Two streams halve the time of the longest query tile, which is what bounds a
 // launch of about one work-group per CU (one long causal sequence); one stream fits two
@@ -879,10 +1110,10 @@ static hipError_t launch_prefill_t(const FwdParams& p, int max_seqlen_q, hipStre
   // given) the longest row's query count, which bounds them for causal self-attention batches.
   const int max_keys = p.S > 0 ? p.S : max_seqlen_q;
   if (prefill_streams(grid, p.n_cus, max_keys) == 1)
-    hipLaunchKernelGGL((fa2_prefill_kernel<E, MODE, 1>), dim3(grid), dim3(PfShape<1>::kThreads), 0,
+    hipLaunchKernelGGL((fa2_prefill_kernel<E, MODE, 1, false, ItemMap>), dim3(grid), dim3(PfShape<1>::kThreads), 0,
                        stream, p, n_qt, map);
   else
-    hipLaunchKernelGGL((fa2_prefill_kernel<E, MODE, 2>), dim3(grid), dim3(PfShape<2>::kThreads), 0,
+    hipLaunchKernelGGL((fa2_prefill_kernel<E, MODE, 2, false, ItemMap>), dim3(grid), dim3(PfShape<2>::kThreads), 0,
                        stream, p, n_qt, map);
   return hipGetLastError();
 }
