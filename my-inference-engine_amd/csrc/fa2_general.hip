@@ -367,8 +367,10 @@ __global__ __launch_bounds__(64 * kGenWaves) void fa2_general_kernel(FwdParams p
 // than CUs (a short sequence with few heads).  A work-group = W waves on the SAME 16 query rows;
 // wave w walks the w-th W-th of the 32-key pairs those rows see, loading its K and V operands
 // straight from global memory (no LDS, no barrier in the loop), and the W waves' (m, l, O) are
-// merged through LDS at the end, each wave finishing every W-th d-block.  W = 4, or 8 (twice the
-// key split) when the grid leaves a whole CU to each work-group (d_v <= 128).
+// merged through LDS at the end.  W = 4, or 8 (twice the key split) when the grid leaves a whole CU
+// to each work-group (d_v <= 128).  Bound by the latency of a pair's loads and, where two
+// work-groups share a CU, by the longer one's chain: wide V loads and pairing long with short tiles
+// took 1 x 12 x 512 x 128 fp32 from 36.0 to 25.9 us, 1 x 12 x 1000 x 256 bf16 from 142 to 87.
 template <class E, int D, int DV, int W>
 __global__ __launch_bounds__(64 * W) void fa2_general_split_kernel(FwdParams p) {
   constexpr int kGenWaves = W;
@@ -380,7 +382,7 @@ __global__ __launch_bounds__(64 * W) void fa2_general_split_kernel(FwdParams p) 
   constexpr int kDB = D / 16, kVB = DV / 16, kDO = D / 32;
   __shared__ float sm_m[kGenWaves][kGenRows];
   __shared__ float sm_l[kGenWaves][kGenRows];
-  __shared__ f32x4 sm_o[kGenWaves][kVB][64];
+  __shared__ float sm_o[kGenWaves][4][kVB][64];   // [wave][element r][d-block][lane]
   const uint32_t wg_linear = blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z);
   probe_mark(p.clock_probe, wg_linear, false);
 
@@ -390,7 +392,11 @@ __global__ __launch_bounds__(64 * W) void fa2_general_split_kernel(FwdParams p) 
   const int hk = h / p.group;
   const int kv_len = p.kv_lens ? clamp_len(p.kv_lens[b], p.S) : p.S;
   const int off = kv_len - p.T;  // query i sits at key position i + off
-  const int q0 = blockIdx.x * kGenRows;
+  // Long and short causal tiles share a CU: work-groups w and w + CUs land on one, so the heads of
+  // every other round of work-groups walk their tiles in the opposite order.
+  const int round = (h + gridDim.y * b) / max(1, p.n_cus / (int)gridDim.x);
+  const int tile = round & 1 ? blockIdx.x : gridDim.x - 1 - blockIdx.x;
+  const int q0 = tile * kGenRows;
   const int q = q0 + n;
   const int q_last = min(q0 + kGenRows, p.T) - 1;
   const int hi = p.causal ? max(0, min(kv_len, q_last + off + 1)) : kv_len;
@@ -421,24 +427,23 @@ __global__ __launch_bounds__(64 * W) void fa2_general_split_kernel(FwdParams p) 
   float m_run = -INFINITY, l_run = 0.f;
   const float c = p.scale_log2;
 
-  // A pair's V^T gathers are issued with its K loads, before the score MFMAs, so that a pair
-  // costs one memory round trip instead of two (when a pair's V fits 512 bytes per row).
-  constexpr bool kVPre = DV * (int)sizeof(T) <= 512;
+  // V^T operands: row m of d-block i is d = kVB * m + i, so that a lane's share of a V row, element m
+  // of every block, is contiguous and comes in the widest loads there are (one key's kVB elements;
+  // element-wise gathers of d = 16 i + m took four to eight times the load instructions).  A pair's
+  // V loads are issued with its K loads, before the score MFMAs, so that a pair costs one memory
+  // round trip.
+  struct alignas(kVB * sizeof(T) < 16 ? kVB * sizeof(T) : 16) VRow { T e[kVB]; };
   for (int pr = pr_lo; pr < pr_hi; ++pr) {
     const int kb = 32 * pr;
-    Quad vpre[kVPre ? kVB : 1][2];
-    if constexpr (kVPre) {
+    VRow vr[2][4];
 #pragma unroll
-      for (int i = 0; i < kVB; ++i)
+    for (int ch = 0; ch < 2; ++ch)
 #pragma unroll
-        for (int ch = 0; ch < 2; ++ch)
-#pragma unroll
-          for (int j = 0; j < 4; ++j) {
-            const int key = kb + 16 * ch + 4 * g + j;
-            const T* vr = vp + (int64_t)min(key, kv_len - 1) * p.v_st + 16 * i + n;
-            vpre[i][ch][j] = key < kv_len ? G::load1(vr) : 0;
-          }
-    }
+      for (int j = 0; j < 4; ++j) {
+        const int key = kb + 16 * ch + 4 * g + j;   // past kv_len: zeros, from a clamped address
+        vr[ch][j] = *reinterpret_cast<const VRow*>(vp + (int64_t)min(key, kv_len - 1) * p.v_st + kVB * n);
+        if (key >= kv_len) vr[ch][j] = VRow{};
+      }
     // S^T of the two 16-key chunks: K as the A operand straight from global memory (rows past
     // kv_len read as zero operands, their address clamped to row 0).
     f32x4 st[2];
@@ -486,24 +491,13 @@ __global__ __launch_bounds__(64 * W) void fa2_general_split_kernel(FwdParams p) 
     }
     l_run = l_run * alpha + ls;
 
-    // V^T as the A operand, gathered from global memory: element j of chunk ch is
-    // V[kb + 16*ch + 4*g + j][16*i + n] (rows past kv_len read as 0, address clamped).
 #pragma unroll
     for (int i = 0; i < kVB; ++i) {
       Quad va[2];
-      if constexpr (kVPre) {
-        va[0] = vpre[i][0];
-        va[1] = vpre[i][1];
-      } else {
 #pragma unroll
-        for (int ch = 0; ch < 2; ++ch)
+      for (int ch = 0; ch < 2; ++ch)
 #pragma unroll
-          for (int j = 0; j < 4; ++j) {
-            const int key = kb + 16 * ch + 4 * g + j;
-            const T* vr = vp + (int64_t)min(key, kv_len - 1) * p.v_st + 16 * i + n;
-            va[ch][j] = key < kv_len ? G::load1(vr) : 0;
-          }
-      }
+        for (int j = 0; j < 4; ++j) va[ch][j] = vr[ch][j].e[i];
       f32x4 acc = oacc[i] * alpha;
       if constexpr (k16) {
         const u32x2 a0 = __builtin_bit_cast(u32x2, va[0]), a1 = __builtin_bit_cast(u32x2, va[1]);
@@ -517,7 +511,8 @@ __global__ __launch_bounds__(64 * W) void fa2_general_split_kernel(FwdParams p) 
     }
   }
 
-  // Merge the 4 waves: lane (n, g) of every wave holds d = 16*i + 4*g + r of query q0 + n.
+  // Merge the waves: lane (n, g) of every wave holds d = kVB (4g + r) + i of query q0 + n in
+  // element r of block i.
   float l_w = l_run + __shfl_xor(l_run, 16);
   l_w += __shfl_xor(l_w, 32);
   if (g == 0) {
@@ -525,7 +520,9 @@ __global__ __launch_bounds__(64 * W) void fa2_general_split_kernel(FwdParams p) 
     sm_l[wave][n] = l_w;
   }
 #pragma unroll
-  for (int i = 0; i < kVB; ++i) sm_o[wave][i][lane] = oacc[i];
+  for (int i = 0; i < kVB; ++i)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) sm_o[wave][r][i][lane] = oacc[i][r];
   __syncthreads();
   float M = sm_m[0][n];
 #pragma unroll
@@ -540,11 +537,19 @@ __global__ __launch_bounds__(64 * W) void fa2_general_split_kernel(FwdParams p) 
   if (q >= p.T) return;
   const float inv = L > 0.f ? 1.f / L : 0.f;
   T* op = reinterpret_cast<T*>(p.o) + b * p.o_sb + h * p.o_sh + (int64_t)q * p.o_st;
-  for (int i = wave; i < kVB; i += kGenWaves) {
-    f32x4 o = sm_o[0][i][lane] * f[0];
+  // wave w finishes element r = w % 4: kVB consecutive dims (with 8 waves, half of them each)
+  constexpr int kHalves = kGenWaves / 4 > 1 && kVB > 1 ? 2 : 1, kPer = kVB / kHalves;
+  if (wave < 4 * kHalves) {
+    struct alignas(kPer * sizeof(T) < 16 ? kPer * sizeof(T) : 16) Part { T e[kPer]; } part;
+    const int r = wave & 3, i0 = (wave >> 2) * kPer;
 #pragma unroll
-    for (int u = 1; u < kGenWaves; ++u) o += sm_o[u][i][lane] * f[u];
-    G::store(op + 16 * i + 4 * g, o * inv);
+    for (int i = 0; i < kPer; ++i) {
+      float o = 0.f;
+#pragma unroll
+      for (int u = 0; u < kGenWaves; ++u) o += sm_o[u][r][i0 + i][lane] * f[u];
+      part.e[i] = G::cvt(o * inv);
+    }
+    *reinterpret_cast<Part*>(op + kVB * (4 * g + r) + i0) = part;
   }
   if (p.lse && wave == 0 && g == 0)
     p.lse[b * p.l_sb + h * p.l_sh + (int64_t)q * p.l_st] =
