@@ -18,8 +18,8 @@ CSRC = PKG / "csrc"
 BUILD = PKG / "_build"
 OUT = PKG / "kernels" / "libmi_fa2.so"
 LIBS = {
-    OUT: ["fa2_prefill.hip", "fa2_decode.hip", "fa2_general.hip", "fa2_merge.hip", "rope_kv.hip",
-          "sample.hip", "step_meta.hip", "model_ops.hip", "fa2_capi.cpp"],
+    OUT: ["fa2_prefill.hip", "fa2_decode.hip", "fa2_general.hip", "fa2_prefill_dims.hip", "fa2_merge.hip",
+          "rope_kv.hip", "sample.hip", "step_meta.hip", "model_ops.hip", "fa2_capi.cpp"],
     PKG / "kernels" / "libmi_model.so": ["linear_rows.hip", "model_capi.cpp"],
 }
 

@@ -1,21 +1,25 @@
 // Forward attention over the rest of the reference's input envelope (kernels/fa2.py:164-214):
 // head dims d (Q, K) and d_v (V, O) that are any powers of two from 16 to 256 and may differ, in
 // bf16, fp16 or fp32.  The MFMA prefill and split-KV decode kernels are built for d = d_v = 128 in
-// bf16 / fp16, the shape the engine runs; this kernel is what every other shape runs on.
+// bf16 / fp16, the shape the engine runs; these kernels are what every other shape runs on.
 //
 // Organisation (gfx950, wave64):
-//   * fa2_general_kernel: a work-group = 4 waves on 64 consecutive query rows (16 per wave) of one
-//     (row, query head).  Each step stages 64 keys of K and V in LDS (16-byte loads, rows padded
-//     by 16 bytes), shared by the 4 waves, two barriers per step; when a step fits 32 KB the next
-//     step's rows are loaded into registers while this one computes.
-//   * fa2_general_split_kernel, for launches that would leave CUs idle (fewer than 64 query rows,
-//     or fewer such work-groups than CUs): the 4 (or 8) waves share 16 query rows and split their
-//     keys, loading K and V operands straight from global memory, and merge (m, l, O) through LDS.
+//   * fa2_general_kernel (16-bit types): a work-group = 4 waves on 64 consecutive query rows (16 per
+//     wave) of one (row, query head).  Each step stages 64 keys of K and V in LDS (16-byte loads, rows
+//     padded by 16 bytes), shared by the 4 waves, two barriers per step; when a step fits 32 KB the
+//     next step's rows are loaded into registers while this one computes.
+//   * fa2_general_split_kernel, for fp32 and for launches that would leave CUs idle (fewer than 64
+//     query rows, or fewer such work-groups than CUs): the 4 (or 8) waves share 16 query rows and
+//     split their keys, loading K and V operands straight from global memory, and merge (m, l, O)
+//     through LDS.
+//   * Larger 16-bit launches at d = d_v = 32, 64 or 256 run on the 128-row kernel of
+//     fa2_prefill_dims.hip (launch_general_t has the rule).
 //   * S^T = K Q^T leaves lane l with query column l%16 and keys 4*(l/16) + r of a 16-key chunk,
 //     which is exactly the B-operand layout of O^T += V^T P^T: P never leaves registers.  16-bit
 //     types run both products on v_mfma_f32_16x16x32 (8 consecutive d per lane for the scores,
 //     d = 16 on 16x16x16; pairs of 16-key chunks for PV), fp32 on four v_mfma_f32_16x16x4_f32 per
-//     16-wide slice.  V^T operands come from ds_read_b64_tr_b16 (16-bit) or 4-byte reads (fp32).
+//     16-wide slice.  V^T operands come from ds_read_b64_tr_b16 (staged) or from the widest loads of
+//     a V row there are (split).
 //   * Online softmax as in kernels/fa2.py:136-150, in the exp2 domain (scale * log2(e) folded into
 //     the scores), the running max and sum per lane; the 4 lanes of a query exchange their max
 //     with two xor shuffles.  P is rounded to the input type before the PV product
@@ -42,7 +46,6 @@ template <> struct Gen<BF16> {
   using Quad = i16x4;
   static __device__ __forceinline__ Quad load(const T* p) { return *reinterpret_cast<const Quad*>(p); }
   static __device__ __forceinline__ Quad zero() { return Quad{0, 0, 0, 0}; }
-  static __device__ __forceinline__ short load1(const T* p) { return (short)*p; }
   static __device__ __forceinline__ f32x4 mma(const Quad& a, const Quad& b, f32x4 c) {
     return __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, b, c, 0, 0, 0);
   }
@@ -73,7 +76,6 @@ template <> struct Gen<FP16> {
   typedef _Float16 h4 __attribute__((ext_vector_type(4)));
   static __device__ __forceinline__ Quad load(const T* p) { return *reinterpret_cast<const Quad*>(p); }
   static __device__ __forceinline__ Quad zero() { return Quad{0, 0, 0, 0}; }
-  static __device__ __forceinline__ short load1(const T* p) { return (short)*p; }
   static __device__ __forceinline__ f32x4 mma(const Quad& a, const Quad& b, f32x4 c) {
     return __builtin_amdgcn_mfma_f32_16x16x16f16(__builtin_bit_cast(h4, a),
                                                  __builtin_bit_cast(h4, b), c, 0, 0, 0);
@@ -101,7 +103,6 @@ template <> struct Gen<F32> {
   using Quad = f32x4;
   static __device__ __forceinline__ Quad load(const T* p) { return *reinterpret_cast<const Quad*>(p); }
   static __device__ __forceinline__ Quad zero() { return Quad{0.f, 0.f, 0.f, 0.f}; }
-  static __device__ __forceinline__ float load1(const T* p) { return *p; }
   // The 16x16x4 MFMA takes one k per lane: element i of every lane's quad is k-slot l/16 of the
   // i-th MFMA, so the four cover the slice (A and B use the same element order).
   static __device__ __forceinline__ f32x4 mma(const Quad& a, const Quad& b, f32x4 c) {
@@ -120,22 +121,14 @@ constexpr int kGenRows = 16;  // query rows per wave
 constexpr int kGenKeys = 64;  // keys staged in LDS per step: 4 chunks of 16
 
 // V^T operand of chunk c, d-block i out of the LDS V tile (row pitch VP): lane (m, g) holds
-// V[16c + 4g + j][16i + m] in element j.  16-bit: one ds_read_b64_tr_b16 (lane 4k+q of a 16-lane
-// group points at row 4g + k, columns 4q..4q+3, and receives column m of the 4 rows); fp32: four
-// 4-byte reads.
+// V[16c + 4g + j][16i + m] in element j.  One ds_read_b64_tr_b16: lane 4k+q of a 16-lane group points
+// at row 4g + k, columns 4q..4q+3, and receives column m of the 4 rows.
 template <class E, int VP>
 __device__ __forceinline__ typename Gen<E>::Quad gen_vt(const typename Gen<E>::T* vl, int c, int i,
                                                         int lane) {
   const int g = lane >> 4, m = lane & 15;
-  if constexpr (sizeof(typename Gen<E>::T) == 2) {
-    const int k = m >> 2, q = m & 3;
-    return __builtin_bit_cast(i16x4, ds_read_tr16(vl + (16 * c + 4 * g + k) * VP + 16 * i + 4 * q));
-  } else {
-    f32x4 r;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) r[j] = vl[(16 * c + 4 * g + j) * VP + 16 * i + m];
-    return r;
-  }
+  const int k = m >> 2, q = m & 3;
+  return __builtin_bit_cast(i16x4, ds_read_tr16(vl + (16 * c + 4 * g + k) * VP + 16 * i + 4 * q));
 }
 
 template <class E, int D, int DV>
@@ -143,10 +136,10 @@ __global__ __launch_bounds__(64 * kGenWaves) void fa2_general_kernel(FwdParams p
   using G = Gen<E>;
   using T = typename G::T;
   using Quad = typename G::Quad;
-  constexpr bool k16 = sizeof(T) == 2;
-  // 16-bit types with d >= 32 take the scores on v_mfma_f32_16x16x32 (8 consecutive d per lane:
-  // 16-byte operands); d = 16 and fp32 on 16-wide slices.
-  constexpr bool kOct = k16 && D >= 32;
+  static_assert(sizeof(T) == 2, "fp32 runs on the split kernel");
+  // d >= 32 takes the scores on v_mfma_f32_16x16x32 (8 consecutive d per lane: 16-byte operands);
+  // d = 16 on 16-wide slices.
+  constexpr bool kOct = D >= 32;
   constexpr int kDB = D / 16, kVB = DV / 16, kDO = D / 32;
   constexpr int kEl16 = 16 / sizeof(T);  // elements per 16-byte chunk
   // LDS rows padded by one 16-byte chunk, so that the 16 rows an operand read touches start on
@@ -319,29 +312,23 @@ __global__ __launch_bounds__(64 * kGenWaves) void fa2_general_kernel(FwdParams p
     }
     l_run = l_run * alpha + ls;
 
-    // O^T += V^T P^T, d-block by d-block.  16-bit: chunks in pairs on v_mfma_f32_16x16x32, k-slots
+    // O^T += V^T P^T, d-block by d-block: chunks in pairs on v_mfma_f32_16x16x32, k-slots
     // 8g + j holding key 4g + j of the first chunk (j < 4) and of the second (j >= 4) in both
     // operands; a pair is skipped when its first chunk is (the second then holds P = 0 rows).
 #pragma unroll
     for (int i = 0; i < kVB; ++i) {
       f32x4 acc = oacc[i] * alpha;
-      if constexpr (k16) {
 #pragma unroll
-        for (int pr2 = 0; pr2 < 2; ++pr2)
-          if (kb + 32 * pr2 < wave_hi) {
-            const i16x4 a0 = gen_vt<E, VP>(vl, 2 * pr2, i, lane);
-            const i16x4 a1 = gen_vt<E, VP>(vl, 2 * pr2 + 1, i, lane);
-            const u32x2 a0w = __builtin_bit_cast(u32x2, a0), a1w = __builtin_bit_cast(u32x2, a1);
-            const u32x2 b0w = __builtin_bit_cast(u32x2, pq[2 * pr2]);
-            const u32x2 b1w = __builtin_bit_cast(u32x2, pq[2 * pr2 + 1]);
-            acc = G::mma8(u32x4{a0w[0], a0w[1], a1w[0], a1w[1]},
-                          u32x4{b0w[0], b0w[1], b1w[0], b1w[1]}, acc);
-          }
-      } else {
-#pragma unroll
-        for (int ch = 0; ch < 4; ++ch)
-          if (kb + 16 * ch < wave_hi) acc = G::mma(gen_vt<E, VP>(vl, ch, i, lane), pq[ch], acc);
-      }
+      for (int pr2 = 0; pr2 < 2; ++pr2)
+        if (kb + 32 * pr2 < wave_hi) {
+          const i16x4 a0 = gen_vt<E, VP>(vl, 2 * pr2, i, lane);
+          const i16x4 a1 = gen_vt<E, VP>(vl, 2 * pr2 + 1, i, lane);
+          const u32x2 a0w = __builtin_bit_cast(u32x2, a0), a1w = __builtin_bit_cast(u32x2, a1);
+          const u32x2 b0w = __builtin_bit_cast(u32x2, pq[2 * pr2]);
+          const u32x2 b1w = __builtin_bit_cast(u32x2, pq[2 * pr2 + 1]);
+          acc = G::mma8(u32x4{a0w[0], a0w[1], a1w[0], a1w[1]},
+                        u32x4{b0w[0], b0w[1], b1w[0], b1w[1]}, acc);
+        }
       oacc[i] = acc;
     }
   }
@@ -557,20 +544,47 @@ __global__ __launch_bounds__(64 * W) void fa2_general_split_kernel(FwdParams p) 
   probe_mark(p.clock_probe, wg_linear, true);  // thread 0's query row always exists
 }
 
-}  // namespace mi_fa2
-
-namespace mi_fa2 {
+// fa2_prefill_dims.hip
+bool prefill_dims_fit(const FwdParams& p, int d);
+hipError_t launch_prefill_dims(const FwdParams& p, int dtype, int d, bool small,
+                               hipStream_t stream);
 
 namespace {
 
 template <class E, int D, int DV>
-hipError_t launch_general_t(const FwdParams& p, hipStream_t stream) {
+hipError_t launch_general_t(const FwdParams& p, int dtype, hipStream_t stream) {
   const int rows_per_wg = kGenWaves * kGenRows;
   const int64_t tiles = (int64_t)((p.T + rows_per_wg - 1) / rows_per_wg) * p.Hq * p.B;
+  constexpr bool k16 = sizeof(typename Gen<E>::T) == 2;
   // Fewer query rows than a work-group holds, or fewer work-groups than the device's CUs (256 on
   // MI355X): split each 16-row tile's keys over 4 waves instead (4x the work-groups, a quarter of
-  // the chain).
-  if (p.T < rows_per_wg || tiles < p.n_cus) {
+  // the chain).  fp32 always: its MFMAs are slow enough to cover the split kernel's loads, and
+  // staging bought nothing (1 x 12 x 1500 x 128 causal: staged 216 us, split 147; 4 x 1500 x 64:
+  // 247 and 218; 4096 x 128: 1,039 and 801).
+  const bool split = !k16 || p.T < rows_per_wg || tiles < p.n_cus;
+  // The sizes of fa2_prefill_dims.hip.  12 heads, causal, us:
+  //  * instead of the split kernel (d <= 64; at d = 256 it is the closer one to 64 bits), where its
+  //    shape of 64 rows gains: by the work, 16-row tiles x keys.  d = 64, split and 64-row: 2 x 300
+  //    (137 K) 8.7 and 9.0, 4 x 200 (125 K) 8.1 and 7.8, 3 x 300 (205 K) 10.3 and 9.2, 1 x 700
+  //    (370 K) 14.2 and 11.0, 1 x 1000 (756 K) 19.2 and 13.5; d = 32 the same within 0.3;
+  //  * instead of the staged kernel, from one full tile of queries on: d = 64, 4 x 64 4.8 staged and
+  //    6.3, 4 x 200 9.0 and 8.3, 4 x 1000 36.7 and 20.9.
+  // Of its two shapes, the 64-row one while its work-groups run at once (d = 32: two per CU) and, where
+  // rows are long, a little beyond; 64-row and 128-row: d = 64, 2 x 400 9.3 and 10.5, 4 x 400 13.7 and
+  // 10.8, 3 x 512 13.8 and 12.2, 1 x 1500 16.7 and 24.5, 2 x 1000 17.5 and 18.7, 2 x 1500 28.5 and 26.7;
+  // d = 32, 4 x 512 8.6 and 9.2, 4 x 1000 15.9 and 15.3.
+  if constexpr (k16 && D == DV && (D == 32 || D == 64 || D == 256)) {
+    const int64_t tiles16 = (int64_t)((p.T + kGenRows - 1) / kGenRows) * p.Hq * p.B;
+    const bool better = split ? D <= 64 && p.T >= kGenRows && tiles16 * p.S >= 150000 : p.T >= 128;
+    if (better && prefill_dims_fit(p, D)) {
+      const bool small = D == 32   ? tiles <= 2 * p.n_cus
+                         : D == 64 ? 4 * tiles <= 3 * p.n_cus ||
+                                         (p.S >= 1000 && 2 * tiles <= 3 * p.n_cus)
+                                   : false;
+      return launch_prefill_dims(p, dtype, D, small, stream);
+    }
+  }
+  if (split) {
     const dim3 grid((p.T + kGenRows - 1) / kGenRows, p.Hq, p.B);
     // Eight waves when every work-group can have a CU of its own (two waves per SIMD): an fp32
     // call of 16 rows x 1 query x 2,048 keys took 114 -> 84 us; with more work-groups than CUs the
@@ -585,31 +599,33 @@ hipError_t launch_general_t(const FwdParams& p, hipStream_t stream) {
     hipLaunchKernelGGL((fa2_general_split_kernel<E, D, DV, 4>), grid, dim3(64 * 4), 0, stream, p);
     return hipGetLastError();
   }
-  const dim3 grid((p.T + rows_per_wg - 1) / rows_per_wg, p.Hq, p.B);
-  hipLaunchKernelGGL((fa2_general_kernel<E, D, DV>), grid, dim3(64 * kGenWaves), 0, stream, p);
+  if constexpr (k16) {
+    const dim3 grid((p.T + rows_per_wg - 1) / rows_per_wg, p.Hq, p.B);
+    hipLaunchKernelGGL((fa2_general_kernel<E, D, DV>), grid, dim3(64 * kGenWaves), 0, stream, p);
+  }
   return hipGetLastError();
 }
 
 template <class E, int D>
-hipError_t launch_general_dv(const FwdParams& p, int dv, hipStream_t stream) {
+hipError_t launch_general_dv(const FwdParams& p, int dtype, int dv, hipStream_t stream) {
   switch (dv) {
-    case 16: return launch_general_t<E, D, 16>(p, stream);
-    case 32: return launch_general_t<E, D, 32>(p, stream);
-    case 64: return launch_general_t<E, D, 64>(p, stream);
-    case 128: return launch_general_t<E, D, 128>(p, stream);
-    case 256: return launch_general_t<E, D, 256>(p, stream);
+    case 16: return launch_general_t<E, D, 16>(p, dtype, stream);
+    case 32: return launch_general_t<E, D, 32>(p, dtype, stream);
+    case 64: return launch_general_t<E, D, 64>(p, dtype, stream);
+    case 128: return launch_general_t<E, D, 128>(p, dtype, stream);
+    case 256: return launch_general_t<E, D, 256>(p, dtype, stream);
   }
   return hipErrorInvalidValue;
 }
 
 template <class E>
-hipError_t launch_general_e(const FwdParams& p, int d, int dv, hipStream_t stream) {
+hipError_t launch_general_e(const FwdParams& p, int dtype, int d, int dv, hipStream_t stream) {
   switch (d) {
-    case 16: return launch_general_dv<E, 16>(p, dv, stream);
-    case 32: return launch_general_dv<E, 32>(p, dv, stream);
-    case 64: return launch_general_dv<E, 64>(p, dv, stream);
-    case 128: return launch_general_dv<E, 128>(p, dv, stream);
-    case 256: return launch_general_dv<E, 256>(p, dv, stream);
+    case 16: return launch_general_dv<E, 16>(p, dtype, dv, stream);
+    case 32: return launch_general_dv<E, 32>(p, dtype, dv, stream);
+    case 64: return launch_general_dv<E, 64>(p, dtype, dv, stream);
+    case 128: return launch_general_dv<E, 128>(p, dtype, dv, stream);
+    case 256: return launch_general_dv<E, 256>(p, dtype, dv, stream);
   }
   return hipErrorInvalidValue;
 }
@@ -620,9 +636,9 @@ hipError_t launch_general_e(const FwdParams& p, int d, int dv, hipStream_t strea
 hipError_t launch_general(const FwdParams& p, int dtype, int d, int dv, hipStream_t stream) {
   if (p.B == 0 || p.T == 0) return hipSuccess;
   switch (dtype) {
-    case 0: return launch_general_e<BF16>(p, d, dv, stream);
-    case 1: return launch_general_e<FP16>(p, d, dv, stream);
-    case 2: return launch_general_e<F32>(p, d, dv, stream);
+    case 0: return launch_general_e<BF16>(p, dtype, d, dv, stream);
+    case 1: return launch_general_e<FP16>(p, dtype, d, dv, stream);
+    case 2: return launch_general_e<F32>(p, dtype, d, dv, stream);
   }
   return hipErrorInvalidValue;
 }

@@ -1,0 +1,71 @@
+"""The prefill kernel for head dims 32, 64 and 256 (csrc/fa2_prefill_dims.hip), at shapes the
+dispatch gives it, against the fp32 oracle; tolerances as for every 16-bit output of the general
+envelope (tests/test_fa2_general_gpu.py)."""
+import math
+
+import pytest
+import torch
+
+from conftest import announce
+from kernels.fa2 import FlashAttention2Function, fa2_forward
+from oracle import sdpa
+from test_fa2_general_gpu import check_close, rand
+
+pytestmark = pytest.mark.gpu
+DTYPES = pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "fp16"])
+
+
+# T, S, heads, kv_lens: a last tile of one row, of 127 and of 128; keys one past, one short of and at a
+# tile; rows with fewer keys than queries, one key and none; more heads than XCDs, one kv head; both
+# shapes (64 and 128 rows per work-group)
+@DTYPES
+@pytest.mark.parametrize("causal", [True, False], ids=["causal", "full"])
+@pytest.mark.parametrize("d", [32, 64, 256])
+@pytest.mark.parametrize("T,S,heads,lens", [
+    (257, 257, (12, 2), [257, 256, 1, 0]), (383, 383, (6, 6), [383, 300, 129, 65]),
+    (384, 640, (20, 1), [640, 641 - 257]), (130, 320, (16, 2), [320, 319, 64, 63] * 2),
+    (200, 100, (12, 2), [100] * 16), (1025, 1100, (12, 2), [1100]),
+    (513, 513, (12, 4), [513, 512, 449, 100])])
+def test_against_the_oracle(T, S, heads, lens, d, causal, dtype):
+    Hq, Hkv = heads
+    B = len(lens)
+    g = torch.Generator().manual_seed(T + S + d)
+    q = torch.randn(B, T, Hq, d, generator=g).to(dtype).transpose(1, 2)   # strided heads
+    k, v = rand((B, Hkv, S, d), g, dtype), rand((B, Hkv, S, d), g, dtype)
+    for b, n in enumerate(lens):   # padding is never read
+        k[b, :, n:] = float("nan")
+        v[b, :, n:] = float("inf")
+    announce(f"[gpu] prefill dims: d={d} T={T} S={S} heads={heads} causal={causal} {dtype}")
+    out, lse = fa2_forward(q.cuda(), k.cuda(), v.cuda(), causal,
+                           torch.tensor(lens, dtype=torch.int32, device="cuda"), return_lse=True)
+    torch.cuda.synchronize()
+    check_close(out, sdpa.attention_ref(q, k, v, causal, lens), dtype, f"d={d}")
+    want = sdpa.lse_ref(q, k.nan_to_num(0.), causal, lens)
+    fin = torch.isfinite(want)
+    assert torch.equal(fin, torch.isfinite(lse.cpu()))
+    # the row sum adds P as rounded for the PV product (unit roundoff 2^-8 at most)
+    assert (lse.cpu()[fin] - want[fin]).abs().max().item() < math.log1p(2.0 ** -8) + 1e-3
+
+
+def test_large_scores_move_the_running_maximum():
+    # each key's score outgrows the one before by far more than the reference may lag (2^8)
+    g = torch.Generator().manual_seed(3)
+    q = torch.ones(4, 12, 300, 64).bfloat16()
+    k = (torch.arange(300).view(1, 1, 300, 1) * torch.ones(4, 2, 300, 64) * 0.25).bfloat16()
+    v = rand((4, 2, 300, 64), g, torch.bfloat16)
+    out = FlashAttention2Function.apply(q.cuda(), k.cuda(), v.cuda(), True, None)
+    # every output is about one V value, so its rounding to bf16 is not small beside the bars: half a
+    # unit is 2^-8 of the value at most and 2^-9 on average
+    ref = sdpa.attention_ref(q, k, v, True)
+    err = (out.float().cpu() - ref).abs()
+    assert (err <= 1e-2 + 2.0 ** -8 * ref.abs()).all()
+    assert err.mean().item() < 1e-3 + 2.0 ** -9 * ref.abs().mean().item()
+
+
+def test_overlapping_key_rows_stay_accepted():
+    # a K whose token stride is 0 (one key expanded) is read by the general kernel, as before
+    q = torch.randn(4, 12, 300, 64, generator=torch.Generator().manual_seed(5)).bfloat16()
+    k = torch.randn(4, 2, 1, 64).bfloat16().cuda().expand(4, 2, 300, 64)
+    v = torch.randn(4, 2, 300, 64, generator=torch.Generator().manual_seed(6)).bfloat16()
+    out = FlashAttention2Function.apply(q.cuda(), k, v.cuda(), True, None)
+    check_close(out, sdpa.attention_ref(q, k.cpu(), v, True), torch.bfloat16, "stride 0")
