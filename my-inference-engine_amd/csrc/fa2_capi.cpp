@@ -10,6 +10,7 @@
 #include <cstdio>
 #include <cstdlib>
 #include <mutex>
+#include <utility>
 
 #include "fa2_common.h"
 
@@ -117,6 +118,43 @@ int plan_of_current_device(Plan* out) {
                 hipGetErrorString(g_plan_err[dev]));
   *out = g_plan[dev];
   return MI_FA2_OK;
+}
+
+// Arrival counters: the last work-group of a launch to reach a counter finishes what the others left
+// in the launch's workspace.  They have to be zero when the launch starts, which a workspace (contents
+// arbitrary) cannot promise and a fill would cost a launch for; these are static device memory, zero
+// when the library is loaded, and every launch leaves them at zero.  Launches that may overlap in time
+// must not share counters, and do not share workspaces: a region belongs to one workspace address on
+// one device, for good.  Null, when the table is full or the call needs more than a region holds (the
+// caller then takes a second launch instead).
+constexpr int kCounterRegions = 128, kCountersPerRegion = 2048;
+static __device__ uint32_t counters[kCounterRegions * kCountersPerRegion];
+
+struct CounterTable {
+  std::mutex mutex;
+  uint32_t* base[kMaxDevices] = {};
+  int used = 0;
+  std::pair<int, const void*> owner[kCounterRegions];
+};
+CounterTable g_counters;
+
+uint32_t* arrival_counters(const void* workspace, int64_t n) {
+  int dev = -1;
+  if (n > kCountersPerRegion || hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kMaxDevices)
+    return nullptr;
+  std::lock_guard<std::mutex> lock(g_counters.mutex);
+  if (!g_counters.base[dev]) {
+    void* at = nullptr;
+    if (hipGetSymbolAddress(&at, HIP_SYMBOL(counters)) != hipSuccess || !at) return nullptr;
+    g_counters.base[dev] = static_cast<uint32_t*>(at);
+  }
+  int r = 0;
+  while (r < g_counters.used && g_counters.owner[r] != std::make_pair(dev, workspace)) ++r;
+  if (r == g_counters.used) {
+    if (r == kCounterRegions) return nullptr;
+    g_counters.owner[g_counters.used++] = {dev, workspace};
+  }
+  return g_counters.base[dev] + (size_t)r * kCountersPerRegion;
 }
 
 // The clock probe set by mi_fa2_set_clock_probe (measurement only; null: off).
@@ -822,8 +860,8 @@ int mi_fa2_sample(int32_t dtype, const void* logits, int64_t row_stride, int32_t
   p.off_lo = (uint32_t)offset;
   p.off_hi = (uint32_t)(offset >> 32);
   if (need) {
-    p.part_s = static_cast<float*>(workspace);
-    p.part_i = reinterpret_cast<int32_t*>(p.part_s + (size_t)batch * p.chunks);
+    p.part = static_cast<uint32_t*>(workspace);
+    p.count = arrival_counters(workspace, batch);
   }
   return launched(mi_fa2::launch_sample(p, dtype, reinterpret_cast<hipStream_t>(stream)));
 }

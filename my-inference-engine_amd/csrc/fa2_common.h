@@ -181,8 +181,8 @@ struct SampleParams {
   const void* logits;
   int64_t row_stride;   // elements
   int32_t* tokens;
-  float* part_s;        // [batch][chunks] best score of each chunk
-  int32_t* part_i;      // [batch][chunks] its index (-1: no candidate)
+  uint32_t* part;       // [batch][chunks][2] best of each chunk: score (fp32 bits), index (-1: none)
+  uint32_t* count;      // [batch] arrival counters, zero between launches, or null
   int batch, vocab, chunks, greedy;
   float inv_t;
   uint32_t seed_lo, seed_hi, off_lo, off_hi;

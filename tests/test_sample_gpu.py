@@ -103,3 +103,22 @@ def test_repeat_calls_are_deterministic_and_offsets_differ():
     a = sample_tokens(logits, 1.0, 1, 0)
     assert torch.equal(a, sample_tokens(logits, 1.0, 1, 0))
     assert (a != sample_tokens(logits, 1.0, 1, 1)).float().mean().item() > 0.5
+
+
+def test_workspaces_beyond_the_counter_table_draw_the_same_tokens():
+    """The arrival counters belong to workspace addresses, a bounded number of them; a call on an
+    address beyond those takes the two-launch path.  Both draw the same tokens."""
+    import ctypes
+    from kernels import _lib
+    lib = _lib.load()
+    g = torch.Generator().manual_seed(8)
+    logits = torch.randn(3, 50000, generator=g).to(torch.bfloat16).to(DEV)
+    want = sample_tokens(logits, 1.0, 11, 5)
+    need = lib.mi_fa2_sample_workspace_size(3, 50000)
+    ws = torch.empty(need + 4 * 200, dtype=torch.uint8, device=DEV)
+    for i in range(200):   # 200 workspaces at 4-byte steps, one call after the other
+        out = torch.full((3,), -7, dtype=torch.int32, device=DEV)
+        _lib.check(lib.mi_fa2_sample(0, logits.data_ptr(), 50000, 3, 50000, 1.0, 11, 5,
+                                     out.data_ptr(), ctypes.c_void_p(ws.data_ptr() + 4 * i), need,
+                                     _lib.stream_of(logits)))
+        assert torch.equal(out, want), i
