@@ -311,6 +311,50 @@ def fa2_paged(q, k_pool, v_pool, block_table, kv_lens, *, block_size=16, max_kv_
     out          optional [B, Hq, T, 128] output (any row/head/token strides, 16-byte aligned)
     Returns O [B, Hq, T, 128] (and the fp32 LSE [B, Hq, T] if return_lse).
     """
+    key = (q.shape, q.stride(), q.dtype, q.device, k_pool.shape, k_pool.stride(), k_pool.dtype,
+           k_pool.device, v_pool.shape, v_pool.stride(), v_pool.dtype, v_pool.device,
+           block_table.shape, block_table.stride(), block_table.dtype, kv_lens.shape, kv_lens.dtype,
+           block_size, max_kv_len, is_causal, return_lse)
+    pl = _PAGED.get(key)
+    if pl is None:
+        pl = _plan_paged(q, k_pool, v_pool, block_table, kv_lens, block_size, max_kv_len, is_causal,
+                         return_lse)
+        if len(_PAGED) >= _MEMO_MAX:
+            _PAGED.clear()
+        _PAGED[key] = pl
+    dtype_code, o_shape, copy_q, q_st, pool_st, o_st, l_st, sizes, tail, ws_bytes = pl
+    kp, vp = k_pool.data_ptr(), v_pool.data_ptr()
+    assert not (kp | vp) & 15, "pools need 16-byte aligned token rows"
+    if copy_q:
+        q = q.contiguous()
+    elif q.data_ptr() & 15:
+        q = _vec(q)
+        q_st = _strides(q)
+    dev = q.device
+    if out is None:
+        O = torch.empty_like(q, memory_format=torch.contiguous_format)
+    else:
+        O = out
+        assert O.shape == o_shape and O.dtype == q.dtype and _dims_ok(O)
+        o_st = _strides(O)
+    L = torch.empty(o_shape[:3], device=dev, dtype=torch.float32) if return_lse else None
+    ws = _workspace(ws_bytes, dev)
+    with _lib.on_device(dev) as stream:
+        _lib.check(_lib.load().mi_fa2_fwd_paged(
+            dtype_code, q.data_ptr(), kp, vp, O.data_ptr(), L.data_ptr() if return_lse else None,
+            block_table.data_ptr(), block_table.stride(0), kv_lens.data_ptr(), *sizes, q_st, pool_st,
+            o_st, l_st, *tail, ws.data_ptr() if ws is not None else None,
+            ws.numel() if ws is not None else 0, stream))
+    return (O, L) if return_lse else O
+
+
+_PAGED = {}
+
+
+def _plan_paged(q, k_pool, v_pool, block_table, kv_lens, block_size, max_kv_len, is_causal,
+                return_lse):
+    """Every check of fa2_paged that its arguments' shapes, strides and types decide, then the
+    launch's constant arguments (base alignment and `out` are checked per call)."""
     assert q.is_cuda and k_pool.is_cuda and v_pool.is_cuda, "q and the pools must be GPU tensors"
     B, Hq, T, d = q.shape
     assert k_pool.dim() == 3 and k_pool.shape == v_pool.shape, "pools are [slots, Hkv, d]"
@@ -328,26 +372,19 @@ def fa2_paged(q, k_pool, v_pool, block_table, kv_lens, *, block_size=16, max_kv_
     # kv_lens are clamped to max_kv_len in-kernel, so this bound keeps every table read in range
     assert 0 <= max_kv_len <= block_table.shape[1] * block_size, \
         "max_kv_len exceeds what the block table can address"
+    assert _strides_ok(k_pool) and _strides_ok(v_pool), "pools need 16-byte aligned token rows"
     if is_causal is None:
         is_causal = T > 1
-    q = _vec(q)
-    assert _dims_ok(k_pool) and _dims_ok(v_pool), "pools need 16-byte aligned token rows"
-    O = out if out is not None else torch.empty((B, Hq, T, d), device=q.device, dtype=q.dtype)
-    assert O.shape == q.shape and O.dtype == q.dtype and _dims_ok(O)
-    L = torch.empty((B, Hq, T), device=q.device, dtype=torch.float32) if return_lse else None
-    lib = _lib.load()
-    ws = _workspace(_paged_ws_bytes(B, Hq, Hkv, T, int(max_kv_len), d), q.device)
-    pool_strides = _pool_strides(k_pool)
-    with _lib.on_device(q.device) as stream:
-        _lib.check(lib.mi_fa2_fwd_paged(
-            _lib.DTYPES[q.dtype], q.data_ptr(), k_pool.data_ptr(), v_pool.data_ptr(), O.data_ptr(),
-            L.data_ptr() if L is not None else None, block_table.data_ptr(), block_table.stride(0),
-            kv_lens.data_ptr(), B, Hq, Hkv, T, int(max_kv_len), d, block_size,
-            k_pool.shape[0] // block_size, _strides(q), pool_strides, _strides(O),
-            _strides(L) if L is not None else None, int(bool(is_causal)),
-            1.0 / math.sqrt(d), ws.data_ptr() if ws is not None else None,
-            ws.numel() if ws is not None else 0, stream))
-    return (O, L) if return_lse else O
+    copy_q = not _strides_ok(q)
+    contig = _contig(q.shape)
+    max_kv_len = int(max_kv_len)
+    return (_lib.DTYPES[q.dtype], q.shape, copy_q,
+            _strides_of(q.shape, contig if copy_q else q.stride()), _pool_strides(k_pool),
+            _strides_of(q.shape, contig),
+            _strides_of(q.shape[:3], _contig(q.shape[:3])) if return_lse else None,
+            (B, Hq, Hkv, T, max_kv_len, d, block_size, k_pool.shape[0] // block_size),
+            (int(bool(is_causal)), 1.0 / math.sqrt(d)),
+            _paged_ws_bytes(B, Hq, Hkv, T, max_kv_len, d))
 
 
 _WS_BYTES = {}

@@ -14,6 +14,7 @@ from . import _lib
 
 DTYPES = {torch.bfloat16: 0, torch.float16: 1, torch.float32: 2}
 
+_WS_BYTES = {}
 _WORKSPACES = {}
 _RETIRED = []   # outgrown buffers: never freed (a captured graph may still use one)
 
@@ -24,7 +25,7 @@ def _workspace(nbytes, device):
     alive, as a graph that captured a call holds its address."""
     if not nbytes:
         return None
-    key = (device, torch.cuda.current_stream(device).cuda_stream)
+    key = (device, torch._C._cuda_getCurrentRawStream(_lib.device_index(device)))
     ws = _WORKSPACES.get(key)
     if ws is None or ws.numel() < nbytes:
         size = int(nbytes)
@@ -48,12 +49,16 @@ def sample_tokens(logits, temperature, seed, offset, out=None):
         out = torch.empty(B, dtype=torch.int32, device=logits.device)
     assert out.dtype == torch.int32 and out.shape == (B,) and out.is_contiguous()
     lib = _lib.load()
-    nbytes = lib.mi_fa2_sample_workspace_size(B, V)
+    nbytes = _WS_BYTES.get((B, V))
+    if nbytes is None:
+        if len(_WS_BYTES) >= 4096:
+            _WS_BYTES.clear()
+        nbytes = _WS_BYTES[B, V] = lib.mi_fa2_sample_workspace_size(B, V)
     ws = _workspace(nbytes, logits.device)
-    with torch.cuda.device(logits.device):
+    with _lib.on_device(logits.device) as stream:
         _lib.check(lib.mi_fa2_sample(
             DTYPES[logits.dtype], logits.data_ptr(), logits.stride(0) if B > 1 else V, B, V,
             float(temperature), int(seed) & (2**64 - 1), int(offset) & (2**64 - 1),
             out.data_ptr(), ws.data_ptr() if ws is not None else None,
-            ws.numel() if ws is not None else 0, _lib.stream_of(logits)))
+            ws.numel() if ws is not None else 0, stream))
     return out
