@@ -31,6 +31,8 @@
 //     key gets O = 0 and LSE = -inf.
 #include "fa2_common.h"
 
+#include <type_traits>
+
 namespace mi_fa2 {
 
 struct F32 {};
@@ -358,7 +360,7 @@ __global__ __launch_bounds__(64 * kGenWaves) void fa2_general_kernel(FwdParams p
 // to each work-group (d_v <= 128).  Bound by the latency of a pair's loads and, where two
 // work-groups share a CU, by the longer one's chain: wide V loads and pairing long with short tiles
 // took 1 x 12 x 512 x 128 fp32 from 36.0 to 25.9 us, 1 x 12 x 1000 x 256 bf16 from 142 to 87.
-template <class E, int D, int DV, int W>
+template <class E, int D, int DV, int W, bool AHEAD>
 __global__ __launch_bounds__(64 * W) void fa2_general_split_kernel(FwdParams p) {
   constexpr int kGenWaves = W;
   using G = Gen<E>;
@@ -420,6 +422,30 @@ __global__ __launch_bounds__(64 * W) void fa2_general_split_kernel(FwdParams p) 
   // V loads are issued with its K loads, before the score MFMAs, so that a pair costs one memory
   // round trip.
   struct alignas(kVB * sizeof(T) < 16 ? kVB * sizeof(T) : 16) VRow { T e[kVB]; };
+  // K operands of a pair, straight from global memory (rows past kv_len are zeros, their address
+  // clamped to row 0).  AHEAD: the next pair's are loaded as soon as this pair's scores are done, so
+  // they travel under the softmax and the PV product.
+  constexpr int kKN = kOct ? kDO : kDB;
+  using KReg = std::conditional_t<kOct, u32x4, Quad>;
+  const auto load_k = [&](int pr, int ch, KReg (&kr)[kKN]) {
+    const int row = 32 * pr + 16 * ch + n;
+    const bool ok = row < kv_len;
+    const T* krow = kp + (int64_t)(ok ? row : 0) * p.k_st;
+#pragma unroll
+    for (int s = 0; s < kKN; ++s) {
+      if constexpr (kOct)
+        kr[s] = ok ? ld16_any(krow + 32 * s + 8 * g) : u32x4{};
+      else
+        kr[s] = ok ? G::load(krow + 16 * s + 4 * g) : G::zero();
+    }
+  };
+  KReg kr[AHEAD ? 2 : 1][kKN];
+  if constexpr (AHEAD) {
+    if (pr_lo < pr_hi) {
+      load_k(pr_lo, 0, kr[0]);
+      load_k(pr_lo, 1, kr[1]);
+    }
+  }
   for (int pr = pr_lo; pr < pr_hi; ++pr) {
     const int kb = 32 * pr;
     VRow vr[2][4];
@@ -431,24 +457,26 @@ __global__ __launch_bounds__(64 * W) void fa2_general_split_kernel(FwdParams p) 
         vr[ch][j] = *reinterpret_cast<const VRow*>(vp + (int64_t)min(key, kv_len - 1) * p.v_st + kVB * n);
         if (key >= kv_len) vr[ch][j] = VRow{};
       }
-    // S^T of the two 16-key chunks: K as the A operand straight from global memory (rows past
-    // kv_len read as zero operands, their address clamped to row 0).
+    // S^T of the two 16-key chunks.
     f32x4 st[2];
 #pragma unroll
     for (int ch = 0; ch < 2; ++ch) {
-      const int kr = kb + 16 * ch + n;
-      const bool k_ok = kr < kv_len;
-      const T* krow = kp + (int64_t)(k_ok ? kr : 0) * p.k_st;
       st[ch] = f32x4{0.f, 0.f, 0.f, 0.f};
-      if constexpr (kOct) {
+      if constexpr (!AHEAD) load_k(pr, ch, kr[0]);
+      const KReg(&ka)[kKN] = kr[AHEAD ? ch : 0];
 #pragma unroll
-        for (int s = 0; s < kDO; ++s)
-          st[ch] = G::mma8(k_ok ? ld16_any(krow + 32 * s + 8 * g) : u32x4{}, qo[s], st[ch]);
-      } else {
-#pragma unroll
-        for (int s = 0; s < kDB; ++s)
-          st[ch] = G::mma(k_ok ? G::load(krow + 16 * s + 4 * g) : G::zero(), qb[s], st[ch]);
+      for (int s = 0; s < kKN; ++s) {
+        if constexpr (kOct) st[ch] = G::mma8(ka[s], qo[s], st[ch]);
+        else st[ch] = G::mma(ka[s], qb[s], st[ch]);
       }
+    }
+    if constexpr (AHEAD) {
+      __builtin_amdgcn_sched_barrier(0);
+      if (pr + 1 < pr_hi) {
+        load_k(pr + 1, 0, kr[0]);
+        load_k(pr + 1, 1, kr[1]);
+      }
+      __builtin_amdgcn_sched_barrier(0);
     }
     float mx = -INFINITY;
 #pragma unroll
@@ -551,6 +579,23 @@ hipError_t launch_prefill_dims(const FwdParams& p, int dtype, int d, bool small,
 
 namespace {
 
+template <class E, int D, int DV, bool AHEAD>
+hipError_t launch_split_t(const FwdParams& p, hipStream_t stream) {
+  const dim3 grid((p.T + kGenRows - 1) / kGenRows, p.Hq, p.B);
+  // Eight waves when every work-group can have a CU of its own (two waves per SIMD): an fp32
+  // call of 16 rows x 1 query x 2,048 keys took 114 -> 84 us; with more work-groups than CUs the
+  // four-wave shape, two work-groups per CU, is faster (1 x 12 x 512 fp32: 35.7 against 37.3 us).
+  if constexpr (DV <= 128) {
+    if ((int64_t)grid.x * grid.y * grid.z <= p.n_cus) {
+      hipLaunchKernelGGL((fa2_general_split_kernel<E, D, DV, 8, AHEAD>), grid, dim3(64 * 8), 0,
+                         stream, p);
+      return hipGetLastError();
+    }
+  }
+  hipLaunchKernelGGL((fa2_general_split_kernel<E, D, DV, 4, AHEAD>), grid, dim3(64 * 4), 0, stream, p);
+  return hipGetLastError();
+}
+
 template <class E, int D, int DV>
 hipError_t launch_general_t(const FwdParams& p, int dtype, hipStream_t stream) {
   const int rows_per_wg = kGenWaves * kGenRows;
@@ -585,19 +630,14 @@ hipError_t launch_general_t(const FwdParams& p, int dtype, hipStream_t stream) {
     }
   }
   if (split) {
-    const dim3 grid((p.T + kGenRows - 1) / kGenRows, p.Hq, p.B);
-    // Eight waves when every work-group can have a CU of its own (two waves per SIMD): an fp32
-    // call of 16 rows x 1 query x 2,048 keys took 114 -> 84 us; with more work-groups than CUs the
-    // four-wave shape, two work-groups per CU, is faster (1 x 12 x 512 fp32: 35.7 against 37.3 us).
-    if constexpr (DV <= 128) {
-      if ((int64_t)grid.x * grid.y * grid.z <= p.n_cus) {
-        hipLaunchKernelGGL((fa2_general_split_kernel<E, D, DV, 8>), grid, dim3(64 * 8), 0, stream,
-                           p);
-        return hipGetLastError();
-      }
-    }
-    hipLaunchKernelGGL((fa2_general_split_kernel<E, D, DV, 4>), grid, dim3(64 * 4), 0, stream, p);
-    return hipGetLastError();
+    // The next pair's K ahead: where two pairs' fit the registers; for fp32 at d = 128, whose waves
+    // then have the whole register file, only on chains long enough to gain by it (1 x 512 26.5 us
+    // without, 34.0 with; 1 x 800 54.4 and 48.8; 1 x 1500 145.7 and 131.9; d = 64, 1 x 512 15.9 and 13.9;
+    // bf16 d = 256, 1 x 1000 83.4 and 64.6).
+    constexpr int kRowBytes = D * (int)sizeof(typename Gen<E>::T);
+    if constexpr (kRowBytes < 512 || k16) return launch_split_t<E, D, DV, true>(p, stream);
+    else if (kRowBytes == 512 && p.S >= 768) return launch_split_t<E, D, DV, kRowBytes == 512>(p, stream);
+    else return launch_split_t<E, D, DV, false>(p, stream);
   }
   if constexpr (k16) {
     const dim3 grid((p.T + rows_per_wg - 1) / rows_per_wg, p.Hq, p.B);
