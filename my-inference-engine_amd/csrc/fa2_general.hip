@@ -449,6 +449,7 @@ __global__ __launch_bounds__(64 * W) void fa2_general_split_kernel(FwdParams p) 
   for (int pr = pr_lo; pr < pr_hi; ++pr) {
     const int kb = 32 * pr;
     VRow vr[2][4];
+    if constexpr (!AHEAD) load_k(pr, 0, kr[0]);   // first: its MFMAs run while V is on its way
 #pragma unroll
     for (int ch = 0; ch < 2; ++ch)
 #pragma unroll
@@ -462,7 +463,9 @@ __global__ __launch_bounds__(64 * W) void fa2_general_split_kernel(FwdParams p) 
 #pragma unroll
     for (int ch = 0; ch < 2; ++ch) {
       st[ch] = f32x4{0.f, 0.f, 0.f, 0.f};
-      if constexpr (!AHEAD) load_k(pr, ch, kr[0]);
+      if constexpr (!AHEAD) {
+        if (ch) load_k(pr, ch, kr[0]);
+      }
       const KReg(&ka)[kKN] = kr[AHEAD ? ch : 0];
 #pragma unroll
       for (int s = 0; s < kKN; ++s) {
