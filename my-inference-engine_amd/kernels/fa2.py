@@ -311,6 +311,12 @@ def fa2_paged(q, k_pool, v_pool, block_table, kv_lens, *, block_size=16, max_kv_
     out          optional [B, Hq, T, 128] output (any row/head/token strides, 16-byte aligned)
     Returns O [B, Hq, T, 128] (and the fp32 LSE [B, Hq, T] if return_lse).
     """
+    # plain values only: the plan is looked up by them
+    if type(max_kv_len) is not int and max_kv_len is not None:
+        max_kv_len = int(max_kv_len)
+    if is_causal is not None:
+        is_causal = bool(is_causal)
+    block_size, return_lse = int(block_size), bool(return_lse)
     key = (q.shape, q.stride(), q.dtype, q.device, k_pool.shape, k_pool.stride(), k_pool.dtype,
            k_pool.device, v_pool.shape, v_pool.stride(), v_pool.dtype, v_pool.device,
            block_table.shape, block_table.stride(), block_table.dtype, kv_lens.shape, kv_lens.dtype,

@@ -371,7 +371,8 @@ class Qwen2ForCausalLM(nn.Module):
 
     def _few_rows_fit(self, res):
         """Whether every layer of a step over res [tokens, hidden] runs on the few-row kernels."""
-        return (1 <= res.shape[0] <= few_rows.MAX_NORM_ROWS and inference(res, *self.parameters())
+        return (1 <= res.shape[0] <= few_rows.MAX_NORM_ROWS
+                and inference(res, *(self.parameters() if torch.is_grad_enabled() else ()))
                 and all(layer.self_attn.few_rows_fit(res, layer.input_layernorm)
                         and layer.mlp.few_rows_fit(res, layer.post_attention_layernorm)
                         for layer in self.layers))

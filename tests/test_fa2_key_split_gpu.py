@@ -101,3 +101,26 @@ def test_paged(T, lens, block):
     want, want_lse = unsplit(q.cuda(), k.cuda(), v.cuda(), True, ln)
     torch.cuda.synchronize()
     check(got, got_lse, want, want_lse, sdpa.attention_ref(q, k, v, True, lens))
+
+
+def test_paged_plans_are_looked_up_by_value():
+    """fa2_paged's checked launch arguments are kept per combination of shapes, strides, types and plain
+    values: a bound held in a tensor counts by its value at each call, and `out` by its own strides."""
+    g = torch.Generator().manual_seed(1)
+    kp, vp = (torch.randn(64 * 16, 2, 128, generator=g).bfloat16().cuda() for _ in range(2))
+    q = torch.randn(2, 12, 1, 128, generator=g).bfloat16().cuda()
+    table = torch.randperm(64, generator=g).int().view(2, 32).cuda()
+    lens = torch.tensor([500, 300], dtype=torch.int32, device="cuda")
+    want = [fa2_paged(q, kp, vp, table, lens, max_kv_len=n) for n in (512, 128)]
+    bound = torch.tensor(512)
+    assert torch.equal(fa2_paged(q, kp, vp, table, lens, max_kv_len=bound), want[0])
+    bound.fill_(128)   # lengths are clamped to it
+    assert torch.equal(fa2_paged(q, kp, vp, table, lens, max_kv_len=bound), want[1])
+    wide = torch.zeros(2, 12, 1, 256, dtype=torch.bfloat16, device="cuda")
+    out = wide[..., 128:]
+    assert fa2_paged(q, kp, vp, table, lens, max_kv_len=512, out=out).data_ptr() == out.data_ptr()
+    assert torch.equal(out, want[0]) and (wide[..., :128] == 0).all()
+    with pytest.raises(AssertionError):
+        fa2_paged(q, kp, vp, table, lens, max_kv_len=513)
+    with pytest.raises(AssertionError):
+        fa2_paged(q, kp, vp, table, lens.long())
