@@ -42,6 +42,14 @@ MI_MODEL_API int mi_model_linear(int32_t dtype, const void* x, int64_t x_stride,
                                  int32_t out_features, int32_t in_features, void* stream);
 
 /*
+ * Rotary tables (model.py:151-155): cos/sin [rows * tokens_per_row, 128] of
+ * float(starts[row] + t) * float(inv_freq[d % 64]), taken in fp32 and rounded; inv_freq [64].
+ */
+MI_MODEL_API int mi_model_rope_table(int32_t dtype, const int32_t* starts, const void* inv_freq,
+                                     void* cos, void* sin, int32_t rows, int32_t tokens_per_row,
+                                     void* stream);
+
+/*
  * The MLP of one layer, out = [residual +] (silu(g) * u) Wd^T with (g | u) = [rmsnorm] x Wgu^T:
  * x, out, residual [rows, hidden], gate_up_w [2 * inter, hidden] (gate rows first), down_w
  * [hidden, inter].  rows <= 64; hidden: a multiple of 32, at most 2048; inter: a multiple of 32.

@@ -44,6 +44,16 @@ struct LinearParams {
   int32_t num_slots, Hq, Hkv;
 };
 
+// Rotary tables of rows that append `T` tokens each from position starts[row] on.
+struct RopeTableParams {
+  const int32_t* starts;     // [rows]
+  const uint16_t* inv_freq;  // [64]
+  uint16_t* cos;             // [rows * T][128]
+  uint16_t* sin;
+  int32_t rows, T;
+};
+hipError_t launch_rope_table(const RopeTableParams& p, int dtype, hipStream_t stream);
+
 // Work-groups that share a tile's K (1 for K <= 2048).
 int linear_splits(int K);
 hipError_t launch_linear_rows(LinearParams p, int dtype, int epi, int n_cus, hipStream_t stream);

@@ -352,6 +352,30 @@ hipError_t launch_rows_e(const LinearParams& p, int epi, int grid, hipStream_t s
 
 }  // namespace
 
+// cos and sin of position x inverse frequency, in fp32 and rounded, as the reference takes them once
+// per step (model.py:151-155): there about eight small launches of 2 to 4 us each, here one.
+template <typename E>
+__global__ __launch_bounds__(64) void rope_table_kernel(const RopeTableParams p) {
+  const int token = blockIdx.x, d = threadIdx.x;
+  const int row = token / p.T;
+  const float a = (float)(p.starts[row] + (token - row * p.T)) * E::lo(p.inv_freq[d]);
+  const uint16_t c = (uint16_t)lr_r<E>(cosf(a)), s = (uint16_t)lr_r<E>(sinf(a));
+  const int64_t at = (int64_t)token * kHeadDim + d;
+  p.cos[at] = c;
+  p.cos[at + kHeadDim / 2] = c;
+  p.sin[at] = s;
+  p.sin[at + kHeadDim / 2] = s;
+}
+
+hipError_t launch_rope_table(const RopeTableParams& p, int dtype, hipStream_t stream) {
+  const dim3 grid(p.rows * p.T);
+  if (dtype == 0)
+    hipLaunchKernelGGL((rope_table_kernel<BF16>), grid, dim3(64), 0, stream, p);
+  else
+    hipLaunchKernelGGL((rope_table_kernel<FP16>), grid, dim3(64), 0, stream, p);
+  return hipGetLastError();
+}
+
 int linear_splits(int K) {
   const int per_group = 32 * kLrSteps * kLrWaves;
   return (K + per_group - 1) / per_group;

@@ -144,6 +144,26 @@ int mi_model_linear(int32_t dtype, const void* x, int64_t x_stride, const void* 
   return launch(p, dtype, mi_fa2::kOut, stream);
 }
 
+int mi_model_rope_table(int32_t dtype, const int32_t* starts, const void* inv_freq, void* cos,
+                        void* sin, int32_t rows, int32_t tokens_per_row, void* stream) {
+  if (int rc = check_dtype(dtype)) return rc;
+  if (rows < 0 || tokens_per_row < 0 || (int64_t)rows * tokens_per_row > (1 << 24))
+    return fail(kInvalid, "bad sizes: rows=%d tokens_per_row=%d (at most 2^24 tokens)", rows,
+                tokens_per_row);
+  if (rows == 0 || tokens_per_row == 0) return ok();
+  if (!starts) return fail(kInvalid, "starts is NULL");
+  if (!inv_freq) return fail(kInvalid, "inv_freq is NULL");
+  if (int rc = check_ptr("cos", cos)) return rc;
+  if (int rc = check_ptr("sin", sin)) return rc;
+  const mi_fa2::RopeTableParams p{starts, static_cast<const uint16_t*>(inv_freq),
+                                  static_cast<uint16_t*>(cos), static_cast<uint16_t*>(sin), rows,
+                                  tokens_per_row};
+  const hipError_t err =
+      mi_fa2::launch_rope_table(p, dtype, reinterpret_cast<hipStream_t>(stream));
+  if (err != hipSuccess) return fail(kLaunch, "kernel launch failed: %s", hipGetErrorString(err));
+  return ok();
+}
+
 size_t mi_model_mlp_workspace_size(int32_t rows, int32_t hidden, int32_t inter) {
   if (rows <= 0 || hidden <= 0 || inter <= 0) return 0;
   return mlp_space(rows, hidden, inter).total;

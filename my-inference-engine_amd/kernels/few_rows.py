@@ -1,6 +1,7 @@
 """Projections of a decode step's few tokens on the HIP kernel (csrc/linear_rows.hip, through
 libmi_model.so, the C ABI in include/mi_model.h), each with what surrounds it in the same launch:
 
+  rope_tables  cos and sin of the step's positions           (model.py:151-155)
   linear     [residual +] ([rmsnorm] x W^T + bias)           (model.py:81-84,107,204-207)
   mlp        [residual +] SwiGLU MLP of [rmsnorm] x          (model.py:112-138; two launches)
   qkv_rope   rmsnorm, q/k/v projection, rotary embedding and the paged cache write (model.py:92,96)
@@ -30,6 +31,7 @@ SIGNATURES = {
     "mi_model_last_error": (ctypes.c_char_p, []),
     "mi_model_linear": (_i32, [_i32, _p, _i64, _p, _f32, _p, _p, _p, _i64, _p, _i64, _i32, _i32,
                                _i32, _p]),
+    "mi_model_rope_table": (_i32, [_i32, _p, _p, _p, _p, _i32, _i32, _p]),
     "mi_model_mlp_workspace_size": (ctypes.c_size_t, [_i32, _i32, _i32]),
     "mi_model_mlp": (_i32, [_i32, _p, _i64, _p, _f32, _p, _p, _p, _i64, _p, _i64, _i32, _i32, _i32,
                             _p, ctypes.c_size_t, _p]),
@@ -126,6 +128,21 @@ def linear(x, w, bias=None, residual=None, norm_weight=None, eps=0.0, out=None):
             else None, float(eps), _weight(w, (N, K), dt),
             _weight(bias, (N,), dt) if bias is not None else None, rp, rs, op, os_, R, N, K, stream))
     return out
+
+
+def rope_tables(starts, T, inv_freq):
+    """starts [B] int32, inv_freq [64] (16-bit) -> cos, sin [B, 1, T, 128] in inv_freq's dtype for
+    positions starts[b] .. starts[b] + T - 1 (model.py:151-155)."""
+    B, dev = starts.shape[0], starts.device
+    assert starts.is_cuda and starts.dtype == torch.int32 and starts.is_contiguous()
+    assert inv_freq.device == dev and inv_freq.dtype in _lib.DTYPES and inv_freq.is_contiguous()
+    assert inv_freq.shape == (HEAD_DIM // 2,)
+    cos, sin = (torch.empty((B, 1, T, HEAD_DIM), device=dev, dtype=inv_freq.dtype) for _ in range(2))
+    with _lib.on_device(dev) as stream:
+        _check(load().mi_model_rope_table(_lib.DTYPES[inv_freq.dtype], starts.data_ptr(),
+                                          inv_freq.data_ptr(), cos.data_ptr(), sin.data_ptr(), B, T,
+                                          stream))
+    return cos, sin
 
 
 def mlp(x, gate_up_w, down_w, residual=None, norm_weight=None, eps=0.0, out=None):

@@ -321,11 +321,25 @@ class Qwen2ForCausalLM(nn.Module):
         metadata living in static device buffers."""
         _, T = input_ids.shape
         x = self.embed_tokens(input_ids)
-        position_ids = meta.starts_dev[:, None] + torch.arange(T, device=x.device)[None, :]
-        cos, sin = self.rope_cos_sin(position_ids, x.dtype)
+        f, starts = self.inv_freq, meta.starts_dev
+        if (x.is_cuda and f.dtype == x.dtype and x.dtype in (torch.bfloat16, torch.float16)
+                and f.shape == (few_rows.HEAD_DIM // 2,) and f.is_contiguous()
+                and f.device == starts.device and starts.dtype == torch.int32
+                and starts.is_contiguous()):
+            cos, sin = few_rows.rope_tables(starts, T, f)
+        else:
+            position_ids = starts[:, None] + torch.arange(T, device=x.device)[None, :]
+            cos, sin = self.rope_cos_sin(position_ids, x.dtype)
         x = self.run_layers(x, cos, sin, cache, meta)
-        x = self.norm(x[:, -1:])
-        return self.lm_head(x)
+        x, w = x[:, -1:], self.embed_tokens.weight
+        rows = x.reshape(-1, x.shape[-1])
+        if (x.is_cuda and rows.shape[0] <= few_rows.MAX_NORM_ROWS and plain(self.norm)
+                and inference(x, w, self.norm.weight)
+                and type(self).lm_head is Qwen2ForCausalLM.lm_head
+                and few_rows.linear_fits(rows, w, self.norm.weight)):
+            return few_rows.linear(rows, w, norm_weight=self.norm.weight,
+                                   eps=self.norm.eps).view(*x.shape[:-1], w.shape[0])
+        return self.lm_head(self.norm(x))
 
     def lm_head(self, x):
         """Tied-embedding logits (model.py:204-207)."""

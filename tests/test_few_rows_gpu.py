@@ -152,3 +152,18 @@ def test_sizes_outside_the_kernel_are_refused():
         few_rows.linear(x, w)
     assert not few_rows.linear_fits(x[:17], w, norm=w[0, :64].contiguous())
     assert not few_rows.linear_fits(x[:, :48][:4].contiguous(), w[:, :48].contiguous())
+
+
+@DTYPES
+@pytest.mark.parametrize("starts,T", [([0], 1), ([5, 0, 40000, 131071], 1), ([7, 1023], 300)])
+def test_rope_tables_equal_the_torch_chain(starts, T, dtype):
+    inv = (1.0 / (1e6 ** (torch.arange(0, 128, 2).float() / 128))).to(dtype).cuda()
+    st = torch.tensor(starts, dtype=torch.int32, device="cuda")
+    cos, sin = few_rows.rope_tables(st, T, inv)
+    pos = st[:, None] + torch.arange(T, device="cuda")[None, :]
+    fr = pos.float()[..., None] * inv[None, None, :]
+    emb = torch.cat((fr, fr), dim=-1)
+    for got, want in ((cos, emb.cos()), (sin, emb.sin())):
+        # one rounding apart where the two libraries' fp32 values straddle a 16-bit boundary
+        err = (got.float() - want[:, None]).abs()
+        assert (err <= U[dtype] * want[:, None].abs() + 1e-6).all(), err.max().item()
