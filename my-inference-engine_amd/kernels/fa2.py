@@ -156,6 +156,24 @@ def _workspace(nbytes, device):
     return ws
 
 
+def _own_workspace(nbytes, device):
+    """The partials of one prefill whose keys are split (two launches): memory of this call alone, from
+    torch's caching allocator in stream order, so that calls of other threads on the same stream, and
+    graphs captured on one stream and replayed on several, never meet in it.  The call runs unsplit
+    without: so it does when there is no memory for it."""
+    if not nbytes:
+        return None
+    try:
+        return torch.empty(nbytes, dtype=torch.uint8, device=device)
+    except torch.OutOfMemoryError:
+        return None
+
+
+def _decodes(T, group, B):
+    """Whether a call runs on the split-KV decode kernel (uses_decode in csrc/fa2_capi.cpp)."""
+    return T == 1 and group <= 16 and B <= 8192
+
+
 class _Padded:
     """The validated launch of one padded-call shape: its checks ran once, its constant arguments
     (sizes, stride arrays, output shapes, which kernel) are built once, and every later call of the
@@ -163,7 +181,7 @@ class _Padded:
 
     Checked per call, not cached: tensor base alignment (16 bytes) and kv_lens."""
     __slots__ = ("fast", "dtype_code", "dev", "o_shape", "l_shape", "copy_q", "copy_k", "copy_v",
-                 "head", "tail", "ws_bytes")
+                 "head", "tail", "ws_bytes", "workspace")
 
 
 _PADDED = {}
@@ -198,6 +216,8 @@ def _plan_padded(Q, K, V, is_causal):
     # a tensor whose strides do not allow 16-byte vector loads goes through a contiguous copy
     pl.copy_q, pl.copy_k, pl.copy_v = (not _strides_ok(t) for t in (Q, K, V))
     lay = lambda t, cp: _strides_of(t.shape, _contig(t.shape) if cp else t.stride())  # noqa: E731
+    pl.workspace = (_workspace if _decodes(seq_len, num_heads // num_kv_heads, batch_size)
+                    else _own_workspace)
     o_st = _strides_of(pl.o_shape, _contig(pl.o_shape))
     l_st = _strides_of(pl.l_shape, _contig(pl.l_shape))
     qs, ks, vs = lay(Q, pl.copy_q), lay(K, pl.copy_k), lay(V, pl.copy_v)
@@ -246,7 +266,7 @@ def _run_padded(Q, K, V, is_causal, kv_lens, want_lse=True):
     lens = kv_lens.data_ptr() if kv_lens is not None else None
     with _lib.on_device(dev) as stream:
         if pl.fast:
-            ws = _workspace(pl.ws_bytes, dev)
+            ws = pl.workspace(pl.ws_bytes, dev)
             _lib.check(lib.mi_fa2_fwd(
                 pl.dtype_code, q.data_ptr(), k.data_ptr(), v.data_ptr(), O.data_ptr(),
                 lp, lens, *pl.head, *tail,
@@ -328,7 +348,7 @@ def fa2_paged(q, k_pool, v_pool, block_table, kv_lens, *, block_size=16, max_kv_
         if len(_PAGED) >= _MEMO_MAX:
             _PAGED.clear()
         _PAGED[key] = pl
-    dtype_code, o_shape, copy_q, q_st, pool_st, o_st, l_st, sizes, tail, ws_bytes = pl
+    dtype_code, o_shape, copy_q, q_st, pool_st, o_st, l_st, sizes, tail, workspace, ws_bytes = pl
     kp, vp = k_pool.data_ptr(), v_pool.data_ptr()
     assert not (kp | vp) & 15, "pools need 16-byte aligned token rows"
     if copy_q:
@@ -344,7 +364,7 @@ def fa2_paged(q, k_pool, v_pool, block_table, kv_lens, *, block_size=16, max_kv_
         assert O.shape == o_shape and O.dtype == q.dtype and _dims_ok(O)
         o_st = _strides(O)
     L = torch.empty(o_shape[:3], device=dev, dtype=torch.float32) if return_lse else None
-    ws = _workspace(ws_bytes, dev)
+    ws = workspace(ws_bytes, dev)
     with _lib.on_device(dev) as stream:
         _lib.check(_lib.load().mi_fa2_fwd_paged(
             dtype_code, q.data_ptr(), kp, vp, O.data_ptr(), L.data_ptr() if return_lse else None,
@@ -390,6 +410,7 @@ def _plan_paged(q, k_pool, v_pool, block_table, kv_lens, block_size, max_kv_len,
             _strides_of(q.shape[:3], _contig(q.shape[:3])) if return_lse else None,
             (B, Hq, Hkv, T, max_kv_len, d, block_size, k_pool.shape[0] // block_size),
             (int(bool(is_causal)), 1.0 / math.sqrt(d)),
+            _workspace if _decodes(T, Hq // Hkv, B) else _own_workspace,
             _paged_ws_bytes(B, Hq, Hkv, T, max_kv_len, d))
 
 
