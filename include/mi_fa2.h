@@ -298,7 +298,10 @@ MI_FA2_API int mi_fa2_rope_kv_write(int32_t dtype, const void* qkv, int64_t qkv_
  *   temperature <= 0: greedy argmax.
  * Ties go to the lowest index; NaN logits never win; a row with no candidate (all -inf or NaN)
  * gets -1 (torch.multinomial raises there).  batch <= 65535.  Needs the workspace that
- * mi_fa2_sample_workspace_size() returns (0 when vocab <= 8192).  Asynchronous on `stream`.
+ * mi_fa2_sample_workspace_size() returns (0 when vocab <= 8192), of any contents; calls that may
+ * overlap in time must not share one.  Asynchronous on `stream`: one launch for up to 2048 rows on
+ * each of the first 128 workspace addresses of the process, for which the library keeps arrival
+ * counters; two launches otherwise, and while `stream` is being captured.
  */
 MI_FA2_API size_t mi_fa2_sample_workspace_size(int32_t batch, int32_t vocab);
 MI_FA2_API int mi_fa2_sample(int32_t dtype, const void* logits, int64_t row_stride, int32_t batch,

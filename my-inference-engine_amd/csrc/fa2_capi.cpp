@@ -123,10 +123,12 @@ int plan_of_current_device(Plan* out) {
 // Arrival counters: the last work-group of a launch to reach a counter finishes what the others left
 // in the launch's workspace.  They have to be zero when the launch starts, which a workspace (contents
 // arbitrary) cannot promise and a fill would cost a launch for; these are static device memory, zero
-// when the library is loaded, and every launch leaves them at zero.  Launches that may overlap in time
-// must not share counters, and do not share workspaces: a region belongs to one workspace address on
-// one device, for good.  Null, when the table is full or the call needs more than a region holds (the
-// caller then takes a second launch instead).
+// when the library is loaded, and every launch leaves them at zero (fa2_arrival.h).  Launches that may
+// overlap in time must not share counters, and do not share workspaces: a region belongs to one
+// workspace address on one device until the process ends.  Null, and the caller takes a second launch
+// instead: when the table is full, when the call needs more than a region holds, and while a graph is
+// being captured, whose replays may overlap with calls that know nothing of it (two graphs captured on
+// one stream hold the same workspace address, and no counter).
 constexpr int kCounterRegions = 128, kCountersPerRegion = 2048;
 static __device__ uint32_t counters[kCounterRegions * kCountersPerRegion];
 
@@ -138,7 +140,13 @@ struct CounterTable {
 };
 CounterTable g_counters;
 
-uint32_t* arrival_counters(const void* workspace, int64_t n) {
+uint32_t* arrival_counters(const void* workspace, int64_t n, hipStream_t stream) {
+  hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(stream, &capture) != hipSuccess) {
+    (void)hipGetLastError();   // the legacy stream while another one captures: the launch reports it
+    return nullptr;
+  }
+  if (capture != hipStreamCaptureStatusNone) return nullptr;
   int dev = -1;
   if (n > kCountersPerRegion || hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kMaxDevices)
     return nullptr;
@@ -861,7 +869,7 @@ int mi_fa2_sample(int32_t dtype, const void* logits, int64_t row_stride, int32_t
   p.off_hi = (uint32_t)(offset >> 32);
   if (need) {
     p.part = static_cast<uint32_t*>(workspace);
-    p.count = arrival_counters(workspace, batch);
+    p.count = arrival_counters(workspace, batch, reinterpret_cast<hipStream_t>(stream));
   }
   return launched(mi_fa2::launch_sample(p, dtype, reinterpret_cast<hipStream_t>(stream)));
 }

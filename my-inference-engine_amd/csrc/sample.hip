@@ -28,6 +28,7 @@
 // wave's best, far wider than the difference between the two, are scored as above.  The winner is
 // the same.  16 rows of 151,936 bf16: 12.1 + 3.8 us in two
 // launches -> 10.0 us in one (one row: 7.0).
+#include "fa2_arrival.h"
 #include "fa2_common.h"
 
 namespace mi_fa2 {
@@ -209,6 +210,7 @@ __global__ __launch_bounds__(kSmpThreads) void sample_chunk_kernel(const SampleP
   // The chunk's winner goes to the workspace.  With counters, the row's last work-group to arrive
   // reduces them: relaxed agent-scope accesses, each coherent by itself, the store waited for before
   // the arrival is counted.  The counter is left at zero.
+  const uint32_t weight = arrival_weight(chunk, p.chunks);
   uint32_t arrived = 0;
   if (lane == 0) {
     uint32_t* at = p.part + 2 * ((int64_t)row * p.chunks + chunk);
@@ -216,16 +218,13 @@ __global__ __launch_bounds__(kSmpThreads) void sample_chunk_kernel(const SampleP
     __hip_atomic_store(at + 1, (uint32_t)best_i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     if (p.count) {
       asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-      arrived = __hip_atomic_fetch_add(p.count + row, 1u, __ATOMIC_RELAXED,
+      arrived = __hip_atomic_fetch_add(p.count + row, weight, __ATOMIC_RELAXED,
                                        __HIP_MEMORY_SCOPE_AGENT);
     }
   }
-  if (!p.count || __builtin_amdgcn_readfirstlane(arrived) != (uint32_t)p.chunks - 1) return;
+  if (!p.count || __builtin_amdgcn_readfirstlane(arrived) + weight != 0) return;
   const int token = reduce_chunks(p, row, lane, true);
-  if (lane == 0) {
-    p.tokens[row] = token;
-    __hip_atomic_store(p.count + row, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  }
+  if (lane == 0) p.tokens[row] = token;
 }
 
 __global__ __launch_bounds__(64) void sample_reduce_kernel(const SampleParams p) {

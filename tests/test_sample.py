@@ -120,3 +120,25 @@ def test_tiny_temperature_is_greedy_and_offsets_give_fresh_draws():
     assert (a == osample.sample(lg, 1.0, 3, 0)).all()
     assert (a != osample.sample(lg, 1.0, 3, 1)).mean() > 0.5
     assert (a != osample.sample(lg, 1.0, 4, 0)).mean() > 0.5
+
+
+def test_arrival_counts_name_the_last_and_end_at_zero(tmp_path):
+    """A launch alone: only its last work-group's add makes the counter 0, in any order.  Launches that
+    overlap on one counter leave it at 0, whatever their sizes."""
+    import ctypes
+    import random
+    from host_rules import rules
+    weight = rules(tmp_path, "fa2_arrival.h", "uint32_t weight(uint32_t i, uint32_t n) "
+                   "{ return mi_fa2::arrival_weight(i, n); }").weight
+    weight.restype = ctypes.c_uint32
+    rng = random.Random(0)
+    for n in (2, 3, 19, 64, 131072):
+        order = [weight(i, n) for i in range(n)]
+        rng.shuffle(order)
+        count = 0
+        for k, w in enumerate(order):
+            count = (count + w) % 2 ** 32
+            assert (count == 0) == (k == n - 1)
+    mixed = [weight(i, n) for n in (19, 19, 2, 7) for i in range(n)]
+    rng.shuffle(mixed)
+    assert sum(mixed) % 2 ** 32 == 0

@@ -4,12 +4,15 @@ Integer results, so the bar is equality: the kernel draws the same token as the 
 every row whose two best race scores are further apart than fp32 rounding of the scores can move
 them (the kernel forms logit / T - ln(-ln U) in fp32); rows inside that margin are counted and
 must be rare.  The distribution is checked separately against softmax(logits / T)."""
+import re
+import sys
+
 import numpy as np
 import pytest
 import torch
 from scipy import stats
 
-from conftest import announce
+from conftest import PKG, announce
 from kernels.sample import sample_tokens
 from oracle import sample as osample
 
@@ -105,9 +108,54 @@ def test_repeat_calls_are_deterministic_and_offsets_differ():
     assert (a != sample_tokens(logits, 1.0, 1, 1)).float().mean().item() > 0.5
 
 
+def test_graphs_hold_no_counters():
+    """A captured call is two launches: graphs captured on one stream share a workspace address, and
+    their replays may overlap with any call on it."""
+    import ctypes
+    g = torch.Generator().manual_seed(6)
+    logits = torch.randn(3, 50000, generator=g).to(torch.bfloat16).to(DEV)
+    want = sample_tokens(logits, 1.0, 11, 5)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph(keep_graph=True)
+    with torch.cuda.graph(graph):
+        out = sample_tokens(logits, 1.0, 11, 5)
+    n = ctypes.c_size_t()
+    hip = ctypes.CDLL("libamdhip64.so.7")
+    assert hip.hipGraphGetNodes(ctypes.c_void_p(graph.raw_cuda_graph()), None, ctypes.byref(n)) == 0
+    assert n.value == 2
+    graph.instantiate()
+    announce("[gpu] sampler in a graph")
+    for _ in range(3):
+        out.fill_(-7)
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, want)
+        assert torch.equal(sample_tokens(logits, 1.0, 11, 5), want)
+
+
+def test_more_rows_than_a_counter_region_take_two_launches():
+    g = torch.Generator().manual_seed(7)
+    rows, vocab = 2049, 8193
+    logits = torch.randn(rows, vocab, generator=g).to(torch.bfloat16)
+    logits[::50, 8192] = 20.0   # the second chunk's only entry wins
+    announce(f"[gpu] sampler {rows} rows of {vocab}")
+    got = sample_tokens(logits.to(DEV), 0.0, 3, 1).cpu()
+    assert torch.equal(got, logits.float().argmax(-1).int())
+    drawn = sample_tokens(logits.to(DEV), 1.0, 3, 1).cpu()
+    # the rows are keyed by their index: the first 2,048 alone take the one-launch path
+    assert torch.equal(drawn[:2048], sample_tokens(logits[:2048].to(DEV), 1.0, 3, 1).cpu())
+
+
 def test_workspaces_beyond_the_counter_table_draw_the_same_tokens():
     """The arrival counters belong to workspace addresses, a bounded number of them; a call on an
-    address beyond those takes the two-launch path.  Both draw the same tokens."""
+    address beyond those takes the two-launch path.  Both draw the same tokens.  In a process of its
+    own: the table is the process's."""
+    import subprocess
+    announce("[gpu] sampler beyond the counter table, in a child process")
+    subprocess.run([sys.executable, __file__], check=True, timeout=100)
+
+
+def _beyond_the_counter_table():
     import ctypes
     from kernels import _lib
     lib = _lib.load()
@@ -115,6 +163,8 @@ def test_workspaces_beyond_the_counter_table_draw_the_same_tokens():
     logits = torch.randn(3, 50000, generator=g).to(torch.bfloat16).to(DEV)
     want = sample_tokens(logits, 1.0, 11, 5)
     need = lib.mi_fa2_sample_workspace_size(3, 50000)
+    regions = re.search(r"kCounterRegions = (\d+)", (PKG / "csrc" / "fa2_capi.cpp").read_text())
+    assert int(regions[1]) < 200
     ws = torch.empty(need + 4 * 200, dtype=torch.uint8, device=DEV)
     for i in range(200):   # 200 workspaces at 4-byte steps, one call after the other
         out = torch.full((3,), -7, dtype=torch.int32, device=DEV)
@@ -122,3 +172,7 @@ def test_workspaces_beyond_the_counter_table_draw_the_same_tokens():
                                      out.data_ptr(), ctypes.c_void_p(ws.data_ptr() + 4 * i), need,
                                      _lib.stream_of(logits)))
         assert torch.equal(out, want), i
+
+
+if __name__ == "__main__":
+    _beyond_the_counter_table()
