@@ -322,7 +322,7 @@ class Qwen2ForCausalLM(nn.Module):
         _, T = input_ids.shape
         x = self.embed_tokens(input_ids)
         f, starts = self.inv_freq, meta.starts_dev
-        if (x.is_cuda and f.dtype == x.dtype and x.dtype in (torch.bfloat16, torch.float16)
+        if (x.is_cuda and self._own("rope_cos_sin") and f.dtype == x.dtype and x.dtype in (torch.bfloat16, torch.float16)
                 and f.shape == (few_rows.HEAD_DIM // 2,) and f.is_contiguous()
                 and f.device == starts.device and starts.dtype == torch.int32
                 and starts.is_contiguous()):
@@ -335,11 +335,14 @@ class Qwen2ForCausalLM(nn.Module):
         rows = x.reshape(-1, x.shape[-1])
         if (x.is_cuda and rows.shape[0] <= few_rows.MAX_NORM_ROWS and plain(self.norm)
                 and inference(x, w, self.norm.weight)
-                and type(self).lm_head is Qwen2ForCausalLM.lm_head
-                and few_rows.linear_fits(rows, w, self.norm.weight)):
+                and self._own("lm_head") and few_rows.linear_fits(rows, w, self.norm.weight)):
             return few_rows.linear(rows, w, norm_weight=self.norm.weight,
                                    eps=self.norm.eps).view(*x.shape[:-1], w.shape[0])
         return self.lm_head(self.norm(x))
+
+    def _own(self, name):
+        """Whether method `name` is this class's, replaced neither in a subclass nor on the instance."""
+        return getattr(self, name) == getattr(Qwen2ForCausalLM, name).__get__(self)
 
     def lm_head(self, x):
         """Tied-embedding logits (model.py:204-207)."""

@@ -1,0 +1,58 @@
+"""When the model's few-token kernels may do its modules' and methods' work without calling them."""
+import pytest
+import torch
+
+from conftest import announce
+from kv_cache import KVCache
+from model import QwenConfig, Qwen2ForCausalLM
+
+pytestmark = pytest.mark.gpu
+CFG = QwenConfig(hidden_size=256, num_layers=2, num_heads=2, num_kv_heads=1, intermediate_size=512,
+                 vocab_size=512)
+
+
+def make(cls=Qwen2ForCausalLM, dtype=torch.bfloat16):
+    model = cls(CFG).cuda().init_random(std=0.05, seed=0).to(dtype).eval().requires_grad_(False)
+    return model
+
+
+def decode(model, steps=3, rows=3):
+    """Logits of a prompt of 40 tokens and of `steps` single-token steps."""
+    cache = KVCache(32, 16, "cuda", next(model.parameters()).dtype, CFG.num_layers, CFG.num_kv_heads,
+                    CFG.head_dim)
+    seqs = [cache.alloc() for _ in range(rows)]
+    g = torch.Generator().manual_seed(1)
+    outs = [model(torch.randint(0, CFG.vocab_size, (rows, 40), generator=g).cuda(), cache, seqs)]
+    for _ in range(steps):
+        outs.append(model(torch.randint(0, CFG.vocab_size, (rows, 1), generator=g).cuda(), cache, seqs))
+    return torch.cat(outs, 1)
+
+
+def override(model, name, change, on_class):
+    """Replace method `name` by one that changes its result; returns the list of its calls."""
+    calls, old = [], getattr(type(model), name)
+
+    def new(self, *args):
+        calls.append(name)
+        return change(old(self, *args))
+    if on_class:
+        model.__class__ = type("Other", (type(model),), {name: new})
+    else:
+        setattr(model, name, new.__get__(model))
+    return calls
+
+
+@pytest.mark.parametrize("on_class", [True, False], ids=["subclass", "instance"])
+@pytest.mark.parametrize("name,change", [
+    ("rope_cos_sin", lambda cs: (cs[0] * 0.5, cs[1] * 0.5)), ("lm_head", lambda y: y + 1)])
+def test_overridden_methods_are_called(name, change, on_class):
+    announce(f"[gpu] model with its own {name}")
+    model = make()
+    plain = decode(model)
+    calls = override(model, name, change, on_class)
+    got = decode(model)
+    assert len(calls) == 4   # the prompt's step and the three decode steps
+    assert not torch.equal(got, plain)
+    if name == "lm_head":
+        # logits of about 1: two roundings, before and after the 1 is added, and of the product
+        assert (got - 1 - plain).abs().max().item() < 4 * 2.0 ** -8 * plain.abs().max().item() + 2.0 ** -7
