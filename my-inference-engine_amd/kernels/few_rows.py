@@ -91,6 +91,12 @@ def weight_fits(w, x, out_features):
             and out_features > 0 and w.shape[1] % 32 == 0 and 0 < w.shape[1] <= MAX_IN)
 
 
+def bias_fits(b, x, out_features):
+    """Whether b is None or a bias of out_features the kernel reads for rows like x."""
+    return b is None or (b.dtype == x.dtype and b.device == x.device and b.shape == (out_features,)
+                         and b.is_contiguous() and b.data_ptr() % 16 == 0)
+
+
 def linear_fits(x, w, norm=None):
     """Whether `linear` takes x [rows, in] and w [out, in] (and norm, an RMSNorm weight)."""
     if norm is not None and not (norm.dtype == x.dtype and norm.device == x.device

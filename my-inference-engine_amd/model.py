@@ -191,6 +191,7 @@ class Attention(nn.Module):
         return (plain(self, norm, qkv, o) and self.cfg.head_dim == few_rows.HEAD_DIM
                 and few_rows.linear_fits(x, qkv.weight, norm.weight)
                 and qkv.weight.shape[0] == self.q_size + 2 * self.kv_size
+                and few_rows.bias_fits(qkv.bias, x, qkv.weight.shape[0])
                 and few_rows.weight_fits(o.weight, x, x.shape[1])
                 and o.weight.shape[1] == self.q_size and o.bias is None)
 

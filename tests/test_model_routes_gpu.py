@@ -28,6 +28,13 @@ def decode(model, steps=3, rows=3):
     return torch.cat(outs, 1)
 
 
+def close(got, want):
+    """The same logits from kernels that sum in another order: a few bf16 roundings apart, which two
+    layers carry on."""
+    assert torch.isfinite(got).all()
+    assert (got - want).abs().max().item() < 0.05 * want.abs().max().item()
+
+
 def override(model, name, change, on_class):
     """Replace method `name` by one that changes its result; returns the list of its calls."""
     calls, old = [], getattr(type(model), name)
@@ -56,3 +63,27 @@ def test_overridden_methods_are_called(name, change, on_class):
     if name == "lm_head":
         # logits of about 1: two roundings, before and after the 1 is added, and of the product
         assert (got - 1 - plain).abs().max().item() < 4 * 2.0 ** -8 * plain.abs().max().item() + 2.0 ** -7
+
+
+def relayout(p, kind):
+    """p's values off a 16-byte boundary, as in one flat buffer of parameters, or with a stride."""
+    if kind == "offset":
+        flat = torch.zeros(p.numel() + 1, dtype=p.dtype, device=p.device)
+        flat[1:] = p.detach().flatten()
+        return flat[1:].view(p.shape)
+    wide = torch.zeros(p.numel(), 2, dtype=p.dtype, device=p.device)
+    wide[:, 0] = p.detach().flatten()
+    return wide[:, 0]
+
+
+@pytest.mark.parametrize("kind", ["offset", "strided"])
+def test_a_bias_the_kernel_cannot_read_goes_through_the_library(kind):
+    announce(f"[gpu] q/k/v bias {kind}")
+    model = make()
+    plain = decode(model)
+    for layer in model.layers:
+        qkv = layer.self_attn.qkv_proj
+        qkv.bias = torch.nn.Parameter(relayout(qkv.bias, kind), requires_grad=False)
+        x = torch.zeros(3, CFG.hidden_size, dtype=qkv.weight.dtype, device="cuda")
+        assert not layer.self_attn.few_rows_fit(x, layer.input_layernorm)
+    close(decode(model), plain)
