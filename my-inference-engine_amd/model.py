@@ -98,10 +98,11 @@ def transposed(weight):
 
 
 def plain(*modules):
-    """Whether the modules are exactly these classes with nothing hooked on, so that a kernel may do
-    their work without calling them."""
+    """Whether the modules are exactly these classes with nothing hooked on and no forward of their
+    own, so that a kernel may do their work without calling them."""
     return (not nn.modules.module._has_any_global_hook()
             and all(type(m) in (nn.Linear, RMSNorm, Attention, MLP, Block)
+                    and "forward" not in vars(m)
                     and not (m._forward_hooks or m._forward_pre_hooks or m._backward_hooks
                              or m._backward_pre_hooks) for m in modules))
 

@@ -87,3 +87,35 @@ def test_a_bias_the_kernel_cannot_read_goes_through_the_library(kind):
         x = torch.zeros(3, CFG.hidden_size, dtype=qkv.weight.dtype, device="cuda")
         assert not layer.self_attn.few_rows_fit(x, layer.input_layernorm)
     close(decode(model), plain)
+
+
+def watch(model, how):
+    """Put something on layer 0 that the fused kernels would miss; returns its calls, if it has any."""
+    layer, calls = model.layers[0], []
+    if how in ("o_proj", "mlp", "post_attention_layernorm"):
+        m = {"o_proj": layer.self_attn.o_proj, "mlp": layer.mlp,
+             "post_attention_layernorm": layer.post_attention_layernorm}[how]
+        m.register_forward_hook(lambda *a: calls.append(how))
+    elif how == "forward":
+        m = layer.mlp.down_proj
+        old = m.forward
+        m.forward = lambda x: calls.append(how) or old(x)
+    elif how == "grad":
+        layer.mlp.down_proj.weight.requires_grad_(True)
+    return calls
+
+
+@pytest.mark.parametrize("how", ["o_proj", "mlp", "post_attention_layernorm", "forward", "grad"])
+def test_watched_layers_are_called(how):
+    announce(f"[gpu] model layers watched by {how}")
+    model = make()
+    x = torch.zeros(3, CFG.hidden_size, dtype=torch.bfloat16, device="cuda")
+    assert model._few_rows_fit(x) and model.layers[0].mlp.few_rows_fit(x)
+    plain = decode(model)
+    calls = watch(model, how)
+    assert not model._few_rows_fit(x)
+    got = decode(model)
+    # (a norm's module is not called on the GPU: the layer's own launches do its work)
+    if how in ("o_proj", "mlp", "forward"):
+        assert len(calls) == 4
+    close(got, plain)
