@@ -38,6 +38,7 @@ from dataclasses import dataclass
 import torch
 import torch.nn as nn
 import torch.nn.functional as F
+from torch.autograd import forward_ad
 
 from kernels import few_rows
 from kernels.fa2 import fa2_paged, fa2_paged_varlen
@@ -108,9 +109,14 @@ def plain(*modules):
 
 
 def inference(*tensors):
-    """Whether nothing would record a gradient or cast the inputs: the fused kernels do neither."""
+    """Whether nothing would record a gradient, cast the inputs or follow the torch operations (forward
+    mode, vmap and other function transforms, tracers, dispatch modes): the fused kernels, launched
+    outside torch, would be missing there."""
     return (not (torch.is_grad_enabled() and any(t.requires_grad for t in tensors))
-            and not torch.is_autocast_enabled("cuda"))
+            and not torch.is_autocast_enabled("cuda")
+            and forward_ad._current_level < 0 and not torch._C._are_functorch_transforms_active()
+            and not torch._C._len_torch_dispatch_stack() and torch._C._get_tracing_state() is None
+            and not torch.compiler.is_compiling())
 
 
 def repeat_kv(x, n_rep):

@@ -119,3 +119,28 @@ def test_watched_layers_are_called(how):
     if how in ("o_proj", "mlp", "forward"):
         assert len(calls) == 4
     close(got, plain)
+
+
+def test_the_head_follows_torch_where_torch_is_followed():
+    """Forward mode, vmap, a dispatch mode and autocast see the head's product as they would any other."""
+    from torch.utils.flop_counter import FlopCounterMode
+    model = make()
+    w = model.embed_tokens.weight
+    x, t = (torch.randn(4, 1, CFG.hidden_size, dtype=torch.bfloat16, device="cuda") for _ in range(2))
+    announce("[gpu] head under forward mode, vmap, a dispatch mode and autocast")
+    with torch.no_grad():
+        want = model.lm_head(x)
+        close(torch.func.vmap(model.lm_head)(x), want)
+        with FlopCounterMode(display=False) as flops:
+            close(model.lm_head(x), want)
+        assert flops.get_total_flops() == 2 * 4 * CFG.hidden_size * CFG.vocab_size
+        with torch.autograd.forward_ad.dual_level():
+            y = model.lm_head(torch.autograd.forward_ad.make_dual(x, t))
+            tangent = torch.autograd.forward_ad.unpack_dual(y).tangent
+            assert tangent is not None
+            close(tangent, t @ w.T)
+        with torch.autocast("cuda", torch.float16):
+            assert model.lm_head(x).dtype == torch.float16
+    grad = x.clone().requires_grad_(True)
+    model.lm_head(grad).sum().backward()
+    assert grad.grad is not None
