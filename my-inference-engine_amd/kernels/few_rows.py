@@ -24,6 +24,7 @@ MAX_ROWS = 64        # tokens per call
 MAX_NORM_ROWS = 16   # with the norm of x in the same launch
 MAX_IN = 2048        # in features (a work-group's waves hold whole rows of x)
 HEAD_DIM = 128
+_PLAIN = (torch.Tensor, torch.nn.Parameter)
 
 _p, _i32, _i64, _f32 = ctypes.c_void_p, ctypes.c_int32, ctypes.c_int64, ctypes.c_float
 # name -> (restype, argtypes); mirrors include/mi_model.h
@@ -84,26 +85,29 @@ def _readable(t):
                                      and t.stride(0) >= t.shape[1])))
 
 
+def _held(t, x):
+    """Whether parameter t is held as the kernels read it for rows like x: x's type and device,
+    contiguous, 16-byte aligned, a plain tensor (no subclass with operations of its own)."""
+    return (type(t) in _PLAIN and t.dtype == x.dtype and t.device == x.device and t.is_contiguous()
+            and t.data_ptr() % 16 == 0)
+
+
 def weight_fits(w, x, out_features):
     """Whether w is an [out_features, in] weight the kernel reads for rows like x."""
-    return (w.dtype == x.dtype and w.device == x.device and w.is_contiguous() and w.dim() == 2
-            and w.data_ptr() % 16 == 0 and w.shape[0] == out_features and out_features % 16 == 0
+    return (_held(w, x) and w.dim() == 2 and w.shape[0] == out_features and out_features % 16 == 0
             and out_features > 0 and w.shape[1] % 32 == 0 and 0 < w.shape[1] <= MAX_IN)
 
 
 def bias_fits(b, x, out_features):
     """Whether b is None or a bias of out_features the kernel reads for rows like x."""
-    return b is None or (b.dtype == x.dtype and b.device == x.device and b.shape == (out_features,)
-                         and b.is_contiguous() and b.data_ptr() % 16 == 0)
+    return b is None or (_held(b, x) and b.shape == (out_features,))
 
 
 def linear_fits(x, w, norm=None):
     """Whether `linear` takes x [rows, in] and w [out, in] (and norm, an RMSNorm weight)."""
-    if norm is not None and not (norm.dtype == x.dtype and norm.device == x.device
-                                 and norm.is_contiguous() and norm.data_ptr() % 16 == 0
-                                 and norm.shape == x.shape[1:]):
+    if norm is not None and not (_held(norm, x) and norm.shape == x.shape[1:]):
         return False
-    return (1 <= x.shape[0] <= (MAX_ROWS if norm is None else MAX_NORM_ROWS)
+    return (type(x) in _PLAIN and 1 <= x.shape[0] <= (MAX_ROWS if norm is None else MAX_NORM_ROWS)
             and x.dtype in _lib.DTYPES and weight_fits(w, x, w.shape[0])
             and w.shape[1] == x.shape[1] and _readable(x))
 
@@ -113,8 +117,7 @@ def mlp_fits(x, gate_up_w, down_w, norm=None):
     hidden, inter = x.shape[1], down_w.shape[1]
     return (linear_fits(x, gate_up_w, norm) and hidden % 16 == 0 and inter % 32 == 0
             and 0 < inter <= 1 << 18 and gate_up_w.shape[0] == 2 * inter
-            and down_w.shape[0] == hidden and down_w.dtype == x.dtype and down_w.device == x.device
-            and down_w.is_contiguous() and down_w.data_ptr() % 16 == 0)
+            and down_w.shape[0] == hidden and _held(down_w, x))
 
 
 def linear(x, w, bias=None, residual=None, norm_weight=None, eps=0.0, out=None):

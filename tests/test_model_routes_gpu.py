@@ -89,6 +89,10 @@ def test_a_bias_the_kernel_cannot_read_goes_through_the_library(kind):
     close(decode(model), plain)
 
 
+class Other(torch.Tensor):
+    """A tensor subclass, as quantized or distributed weights are."""
+
+
 def watch(model, how):
     """Put something on layer 0 that the fused kernels would miss; returns its calls, if it has any."""
     layer, calls = model.layers[0], []
@@ -102,10 +106,15 @@ def watch(model, how):
         m.forward = lambda x: calls.append(how) or old(x)
     elif how == "grad":
         layer.mlp.down_proj.weight.requires_grad_(True)
+    elif how == "subclass":
+        w = layer.mlp.down_proj.weight
+        layer.mlp.down_proj.weight = torch.nn.Parameter(w.detach().as_subclass(Other),
+                                                        requires_grad=False)
     return calls
 
 
-@pytest.mark.parametrize("how", ["o_proj", "mlp", "post_attention_layernorm", "forward", "grad"])
+@pytest.mark.parametrize("how", ["o_proj", "mlp", "post_attention_layernorm", "forward", "grad",
+                                 "subclass"])
 def test_watched_layers_are_called(how):
     announce(f"[gpu] model layers watched by {how}")
     model = make()
