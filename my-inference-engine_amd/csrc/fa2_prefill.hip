@@ -884,11 +884,15 @@ __global__ __launch_bounds__(256) void fa2_prefill_combine_kernel(const FwdParam
     f32x4 o[kBatch][4];
 #pragma unroll
     for (int u = 0; u < kBatch; ++u) {
+      // a slot past the wave's pieces weighs nothing: zeros, not a piece's sums times 0, which are NaN
+      // where a value is inf
+      const bool live = s0 + u < s_hi;
       const float* q = part + min(s0 + u, s_hi - 1) * stride;
-      m[u] = s0 + u < s_hi ? q[m_at] : -INFINITY;
-      l[u] = q[m_at + kPfRows];
+      m[u] = live ? q[m_at] : -INFINITY;
+      l[u] = live ? q[m_at + kPfRows] : 0.f;
 #pragma unroll
-      for (int k = 0; k < 4; ++k) o[u][k] = *reinterpret_cast<const f32x4*>(q + o_at + k * 256);
+      for (int k = 0; k < 4; ++k)
+        o[u][k] = live ? *reinterpret_cast<const f32x4*>(q + o_at + k * 256) : f32x4{0.f, 0.f, 0.f, 0.f};
     }
     float Mn = M;
 #pragma unroll

@@ -74,6 +74,27 @@ def test_padded(T, heads, lens, causal, dtype):
     check(got, got_lse, want, want_lse, sdpa.attention_ref(q, k, v, causal, lens))
 
 
+@pytest.mark.parametrize("T", [5, 64, 150])
+def test_infinite_values_stay_infinite(T):
+    """An inf in a V row every query sees (an overflow in fp16, say) is an inf of its column, whichever
+    piece holds it."""
+    S, cols = 3001, range(0, 3001, 100)
+    assert ws_bytes(1, 12, 2, T, S) > 0
+    g = torch.Generator().manual_seed(T)
+    q = torch.randn(1, 12, T, 128, generator=g).half()
+    k, v = (torch.randn(1, 2, S, 128, generator=g).half() for _ in range(2))
+    for i, key in enumerate(cols):
+        v[0, :, key, i] = float("inf")
+    announce(f"[gpu] split with infinite values T={T}")
+    qd, kd, vd = q.cuda(), k.cuda(), v.cuda()
+    ln = torch.tensor([S], dtype=torch.int32, device="cuda")
+    got, _ = fa2_forward(qd, kd, vd, False, ln, return_lse=True)
+    want, _ = unsplit(qd, kd, vd, False, ln)
+    torch.cuda.synchronize()
+    assert torch.isinf(want[..., :len(cols)]).all() and torch.isfinite(want[..., len(cols):]).all()
+    assert torch.equal(torch.isinf(got), torch.isinf(want)) and not torch.isnan(got).any()
+
+
 @pytest.mark.parametrize("T,lens,block", [(150, [3001], 16), (5, [7777], 16), (90, [2000, 1999], 32),
                                           (60, [4100, 300], 512), (3, [1300, 2], 128)])
 def test_paged(T, lens, block):
