@@ -28,6 +28,7 @@ power-of-two d and d_v; fp32 inputs with fp32 dots, kernels/fa2.py:129,147) up t
 else is rejected with an AssertionError, never silently computed another way.
 """
 import math
+import operator
 
 import torch
 
@@ -333,10 +334,15 @@ def fa2_paged(q, k_pool, v_pool, block_table, kv_lens, *, block_size=16, max_kv_
     """
     # plain values only: the plan is looked up by them
     if type(max_kv_len) is not int and max_kv_len is not None:
+        # the bound as given: rounding comes after
+        assert 0 <= max_kv_len <= block_table.shape[1] * block_size, \
+            "max_kv_len exceeds what the block table can address"
         max_kv_len = int(max_kv_len)
     if is_causal is not None:
         is_causal = bool(is_causal)
-    block_size, return_lse = int(block_size), bool(return_lse)
+    if type(block_size) is not int:
+        block_size = operator.index(block_size)   # an integer of another type; a float is refused
+    return_lse = bool(return_lse)
     key = (q.shape, q.stride(), q.dtype, q.device, k_pool.shape, k_pool.stride(), k_pool.dtype,
            k_pool.device, v_pool.shape, v_pool.stride(), v_pool.dtype, v_pool.device,
            block_table.shape, block_table.stride(), block_table.dtype, kv_lens.shape, kv_lens.dtype,

@@ -332,3 +332,17 @@ def test_noalloc_paged_forward_refuses_more_than_its_scratch_before_launching():
     assert rc == 3
     msg = lib.mi_fa2_last_error().decode()
     assert "at most 33554432" in msg and str(need) in msg
+
+
+@pytest.mark.parametrize("bad,error", [
+    (dict(block_size=16.5), TypeError), (dict(block_size=16.0), TypeError),
+    (dict(block_size="16"), TypeError), (dict(max_kv_len=-0.5), AssertionError),
+    (dict(max_kv_len=512.5), AssertionError), (dict(max_kv_len=float("nan")), AssertionError),
+    (dict(max_kv_len=torch.tensor(513)), AssertionError)])
+def test_paged_plans_refuse_what_is_no_size(bad, error):
+    # a plan is looked up by plain values; what a value was rounded from is checked before it is rounded
+    from test_split_workspace import on_gpu
+    q, pool = on_gpu(1, 4, 3, 128), on_gpu(512, 2, 128)
+    table, lens = torch.zeros(1, 32, dtype=torch.int32), torch.zeros(1, dtype=torch.int32)
+    with pytest.raises(error):
+        fa2.fa2_paged(q, pool, pool, table, lens, **bad)
