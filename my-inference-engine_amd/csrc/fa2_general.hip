@@ -13,7 +13,7 @@
 //     split their keys, loading K and V operands straight from global memory, and merge (m, l, O)
 //     through LDS.
 //   * Larger 16-bit launches at d = d_v = 32, 64 or 256 run on the 128-row kernel of
-//     fa2_prefill_dims.hip (launch_general_t has the rule).
+//     fa2_prefill_dims.hip (fa2_general_rule.h has the rule).
 //   * S^T = K Q^T leaves lane l with query column l%16 and keys 4*(l/16) + r of a 16-key chunk,
 //     which is exactly the B-operand layout of O^T += V^T P^T: P never leaves registers.  16-bit
 //     types run both products on v_mfma_f32_16x16x32 (8 consecutive d per lane for the scores,
@@ -30,6 +30,7 @@
 //     kv_len, so padding contents (even inf / NaN) never reach the output.  A query that sees no
 //     key gets O = 0 and LSE = -inf.
 #include "fa2_common.h"
+#include "fa2_general_rule.h"
 
 #include <type_traits>
 
@@ -576,7 +577,6 @@ __global__ __launch_bounds__(64 * W) void fa2_general_split_kernel(FwdParams p) 
 }
 
 // fa2_prefill_dims.hip
-bool prefill_dims_fit(const FwdParams& p, int d);
 hipError_t launch_prefill_dims(const FwdParams& p, int dtype, int d, bool small,
                                hipStream_t stream);
 
@@ -601,38 +601,12 @@ hipError_t launch_split_t(const FwdParams& p, hipStream_t stream) {
 
 template <class E, int D, int DV>
 hipError_t launch_general_t(const FwdParams& p, int dtype, hipStream_t stream) {
-  const int rows_per_wg = kGenWaves * kGenRows;
-  const int64_t tiles = (int64_t)((p.T + rows_per_wg - 1) / rows_per_wg) * p.Hq * p.B;
   constexpr bool k16 = sizeof(typename Gen<E>::T) == 2;
-  // Fewer query rows than a work-group holds, or fewer work-groups than the device's CUs (256 on
-  // MI355X): split each 16-row tile's keys over 4 waves instead (4x the work-groups, a quarter of
-  // the chain).  fp32 always: its MFMAs are slow enough to cover the split kernel's loads, and
-  // staging bought nothing (1 x 12 x 1500 x 128 causal: staged 216 us, split 147; 4 x 1500 x 64:
-  // 247 and 218; 4096 x 128: 1,039 and 801).
-  const bool split = !k16 || p.T < rows_per_wg || tiles < p.n_cus;
-  // The sizes of fa2_prefill_dims.hip.  12 heads, causal, us:
-  //  * instead of the split kernel (d <= 64; at d = 256 it is the closer one to 64 bits), where its
-  //    shape of 64 rows gains: by the work, 16-row tiles x keys.  d = 64, split and 64-row: 2 x 300
-  //    (137 K) 8.7 and 9.0, 4 x 200 (125 K) 8.1 and 7.8, 3 x 300 (205 K) 10.3 and 9.2, 1 x 700
-  //    (370 K) 14.2 and 11.0, 1 x 1000 (756 K) 19.2 and 13.5; d = 32 the same within 0.3;
-  //  * instead of the staged kernel, from one full tile of queries on: d = 64, 4 x 64 4.8 staged and
-  //    6.3, 4 x 200 9.0 and 8.3, 4 x 1000 36.7 and 20.9.
-  // Of its two shapes, the 64-row one while its work-groups run at once (d = 32: two per CU) and, where
-  // rows are long, a little beyond; 64-row and 128-row: d = 64, 2 x 400 9.3 and 10.5, 4 x 400 13.7 and
-  // 10.8, 3 x 512 13.8 and 12.2, 1 x 1500 16.7 and 24.5, 2 x 1000 17.5 and 18.7, 2 x 1500 28.5 and 26.7;
-  // d = 32, 4 x 512 8.6 and 9.2, 4 x 1000 15.9 and 15.3.
-  if constexpr (k16 && D == DV && (D == 32 || D == 64 || D == 256)) {
-    const int64_t tiles16 = (int64_t)((p.T + kGenRows - 1) / kGenRows) * p.Hq * p.B;
-    const bool better = split ? D <= 64 && p.T >= kGenRows && tiles16 * p.S >= 150000 : p.T >= 128;
-    if (better && prefill_dims_fit(p, D)) {
-      const bool small = D == 32   ? tiles <= 2 * p.n_cus
-                         : D == 64 ? 4 * tiles <= 3 * p.n_cus ||
-                                         (p.S >= 1000 && 2 * tiles <= 3 * p.n_cus)
-                                   : false;
-      return launch_prefill_dims(p, dtype, D, small, stream);
-    }
-  }
-  if (split) {
+  const GeneralKernel kernel =
+      general_kernel({p.B, p.Hq, p.Hkv, p.T, p.S, p.k_st, p.v_st, D, DV, k16, p.scale_log2, p.n_cus});
+  if (kernel == kGenDims || kernel == kGenDimsSmall)
+    return launch_prefill_dims(p, dtype, D, kernel == kGenDimsSmall, stream);
+  if (kernel == kGenSplit) {
     // The next pair's K ahead: where two pairs' fit the registers; for fp32 at d = 128, whose waves
     // then have the whole register file, only on chains long enough to gain by it (1 x 512 26.5 us
     // without, 34.0 with; 1 x 800 54.4 and 48.8; 1 x 1500 145.7 and 131.9; d = 64, 1 x 512 15.9 and 13.9;
@@ -643,7 +617,8 @@ hipError_t launch_general_t(const FwdParams& p, int dtype, hipStream_t stream) {
     else return launch_split_t<E, D, DV, false>(p, stream);
   }
   if constexpr (k16) {
-    const dim3 grid((p.T + rows_per_wg - 1) / rows_per_wg, p.Hq, p.B);
+    constexpr int kRows = kGenWaves * kGenRows;
+    const dim3 grid((p.T + kRows - 1) / kRows, p.Hq, p.B);
     hipLaunchKernelGGL((fa2_general_kernel<E, D, DV>), grid, dim3(64 * kGenWaves), 0, stream, p);
   }
   return hipGetLastError();

@@ -324,13 +324,6 @@ __global__ __launch_bounds__(
   probe_mark(p.clock_probe, blockIdx.x, true);
 }
 
-// Whether launch_prefill_dims takes the call: K/V rows that neither overlap nor outgrow the loads'
-// 32-bit offsets.
-bool prefill_dims_fit(const FwdParams& p, int d) {
-  const auto stride_ok = [&](int64_t st) { return st >= d && st < (int64_t(1) << 23); };
-  return p.S > 0 && stride_ok(p.k_st) && stride_ok(p.v_st);
-}
-
 template <typename E, int D, int RG, int NS>
 static hipError_t launch_dims_t(const FwdParams& p, hipStream_t stream) {
   using Sh = PdShape<D, RG, NS>;
@@ -349,7 +342,8 @@ static hipError_t launch_dims_e(const FwdParams& p, int d, bool small, hipStream
   return launch_dims_t<E, 256, 4, 1>(p, stream);
 }
 
-// small: the 64-row shape of four key streams (d <= 64).
+// small: the 64-row shape of four key streams (d <= 64).  The calls that fit are
+// fa2_general_rule.h's.
 hipError_t launch_prefill_dims(const FwdParams& p, int dtype, int d, bool small,
                                hipStream_t stream) {
   return dtype == 0 ? launch_dims_e<BF16>(p, d, small, stream)

@@ -7,6 +7,7 @@ import pytest
 import torch
 
 from conftest import announce
+from kernels import _lib
 from kernels.fa2 import FlashAttention2Function, fa2_forward
 from oracle import sdpa
 from test_fa2_general_gpu import check_close, rand
@@ -69,3 +70,19 @@ def test_overlapping_key_rows_stay_accepted():
     v = torch.randn(4, 2, 300, 64, generator=torch.Generator().manual_seed(6)).bfloat16()
     out = FlashAttention2Function.apply(q.cuda(), k, v.cuda(), True, None)
     check_close(out, sdpa.attention_ref(q, k.cpu(), v, True), torch.bfloat16, "stride 0")
+
+
+@pytest.mark.parametrize("d", [32, 64, 256])
+@pytest.mark.parametrize("B,T", [(1, 1000), (4, 1000)])
+@pytest.mark.parametrize("scale", [-0.125, 0.0])
+def test_scales_that_are_not_positive(scale, B, T, d):
+    """Negative: the smallest score weighs most; zero: the mean of the visible values."""
+    g = torch.Generator().manual_seed(d + T)
+    q, k, v = (torch.randn(B, n, T, d, generator=g).bfloat16().cuda() for n in (12, 2, 2))
+    o = torch.full_like(q, float("nan"))
+    announce(f"[gpu] general entry point, scale {scale}, {B} x {T} x {d}")
+    _lib.check(_lib.load().mi_fa2_fwd_general(
+        0, q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), None, None, B, 12, 2, T, T, d, d,
+        *(_lib.strides(t) for t in (q, k, v, o)), None, 1, scale, _lib.stream_of(q)))
+    qs = q.float().cpu() * (scale * math.sqrt(d))   # the oracle scales by 1 / sqrt(d)
+    check_close(o, sdpa.attention_ref(qs, k.float().cpu(), v.float().cpu(), True), torch.bfloat16, "scale")
