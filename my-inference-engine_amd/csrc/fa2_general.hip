@@ -603,7 +603,8 @@ template <class E, int D, int DV>
 hipError_t launch_general_t(const FwdParams& p, int dtype, hipStream_t stream) {
   constexpr bool k16 = sizeof(typename Gen<E>::T) == 2;
   const GeneralKernel kernel =
-      general_kernel({p.B, p.Hq, p.Hkv, p.T, p.S, p.k_st, p.v_st, D, DV, k16, p.scale_log2, p.n_cus});
+      general_kernel({p.B, p.Hq, p.Hkv, p.T, p.S, p.k_st, p.v_st, D, DV, k16, p.scale_log2, p.n_cus,
+                      p.xcd_log2});
   if (kernel == kGenDims || kernel == kGenDimsSmall)
     return launch_prefill_dims(p, dtype, D, kernel == kGenDimsSmall, stream);
   if (kernel == kGenSplit) {

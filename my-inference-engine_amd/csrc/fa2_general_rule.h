@@ -17,16 +17,20 @@ struct GeneralCall {
   int d, dv;
   bool bits16;
   float scale_log2;
-  int n_cus;
+  int n_cus, xcd_log2;
 };
 
 // Whether fa2_prefill_dims_kernel can run the call: K/V rows that neither overlap nor outgrow the
-// loads' 32-bit offsets, and a scale under which the largest score is the largest exponent (its masked
-// scores are -inf before the scaling; the other kernels mask after it and take any).
-inline bool prefill_dims_fit(const GeneralCall& c) {
+// loads' 32-bit offsets; a scale under which the largest score is the largest exponent (its masked
+// scores are -inf before the scaling; the other kernels mask after it and take any); and a launch of
+// one dimension that HIP and the kernel's divisions take: fewer than 2^32 threads.
+inline bool prefill_dims_fit(const GeneralCall& c, bool small) {
   const auto stride_ok = [&](int64_t st) { return st >= c.d && st < (int64_t(1) << 23); };
   if (c.seqlen_k <= 0 || !stride_ok(c.k_stride) || !stride_ok(c.v_stride)) return false;
-  return c.scale_log2 > 0.f && c.scale_log2 < 3.0e38f;
+  if (!(c.scale_log2 > 0.f && c.scale_log2 < 3.0e38f)) return false;
+  const int64_t rows = small ? 64 : 128, threads = c.d > 64 ? 256 : 512, X = int64_t(1) << c.xcd_log2;
+  const int64_t groups = ((c.batch * c.heads_kv) | 1) * ((c.seqlen_q + rows - 1) / rows);
+  return (groups + X - 1) / X * X * (c.heads_q / c.heads_kv) * threads < int64_t(1) << 32;
 }
 
 inline GeneralKernel general_kernel(const GeneralCall& c) {
@@ -58,7 +62,7 @@ inline GeneralKernel general_kernel(const GeneralCall& c) {
                        : c.d == 64 ? 4 * tiles <= 3 * c.n_cus ||
                                          (c.seqlen_k >= 1000 && 2 * tiles <= 3 * c.n_cus)
                                    : false;
-    if (better && prefill_dims_fit(c)) return small ? kGenDimsSmall : kGenDims;
+    if (better && prefill_dims_fit(c, small)) return small ? kGenDimsSmall : kGenDims;
   }
   return split ? kGenSplit : kGenStaged;
 }

@@ -27,3 +27,16 @@ def test_scales_and_strides_the_prefill_kernel_cannot_take(d, B, T):
         assert kernel(B, 12, 2, T, T, d, strides=st) in (SPLIT, STAGED)
     assert kernel(B, 12, 2, T, T, d, strides=((1 << 23) - 8, 4 * d)) == usual
     assert kernel(B, 12, 2, T, 0, d) in (SPLIT, STAGED)
+
+
+@pytest.mark.parametrize("d,threads,rows", [(32, 512, 128), (64, 512, 128), (256, 256, 128)])
+def test_launches_of_one_dimension_stay_below_2_32_threads(d, threads, rows):
+    """HIP refuses a dimension of 2^32 threads; the staged kernel's three-dimensional grid takes as many
+    work-groups as a call may have (65,535 x 65,535 heads)."""
+    most = 2 ** 32 // threads            # work-groups
+    heads = -(-most // 65535)            # of 65,535 rows: just too many
+    for kv_heads in (1, heads):
+        assert kernel(65535, heads, kv_heads, rows, rows, d) == STAGED
+        assert kernel(32768, heads, kv_heads, 2 * rows + 1, rows, d) == STAGED
+        assert kernel(65535, heads - 2, 1 if kv_heads == 1 else heads - 2, rows, rows, d) == DIMS
+    assert kernel(65535, heads - 2, 1, rows, rows, d, xcd_log2=0) == DIMS
