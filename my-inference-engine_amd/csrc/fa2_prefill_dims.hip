@@ -177,6 +177,8 @@ __global__ __launch_bounds__(
     for (int r = 2; r < 16; r += 2) mx = fmax3(mx, s[r], s[r + 1]);
     return mx;
   };
+  constexpr float kExactScore = 0x1p24f;
+  bool exact = false;   // whether some row's maximum is that large (exps)
   const auto move_max = [&](float mx) {
     mx = fmaxf(mx, __shfl_xor(mx, 32)) * c;
     if (__any(mx > m_run)) {
@@ -188,17 +190,31 @@ __global__ __launch_bounds__(
 #pragma unroll
       for (int i = 0; i < kDB; ++i) oacc[i] *= alpha;
       m_run = m_new;
+      exact = __any(m_run != -INFINITY && fabsf(m_run) >= kExactScore);
     }
   };
-  // P^T of 32 keys as the B operand of two k-steps; the row sum adds P as rounded.
+  // P^T of 32 keys as the B operand of two k-steps; the row sum adds P as rounded.  The exponents are
+  // one fma each: the row's largest is then off 0 by the rounding of m_run, which cancels in the
+  // division while it is small (below 1/2 up to kExactScore).  Beyond, where it would overflow, the
+  // products are rounded as m_run was, so that the largest is 0.
   const auto exps = [&](const f32x16& s, u32x4 (&pb)[2]) {
     const float m_use = m_run == -INFINITY ? 0.f : m_run;
     float lt = 0.f;
+    if (exact) {
+#pragma clang fp contract(off)
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      pb[i >> 2][i & 3] = E::pack2(exp2_fast(__builtin_fmaf(s[2 * i], c, -m_use)),
-                                   exp2_fast(__builtin_fmaf(s[2 * i + 1], c, -m_use)));
-      lt = E::sum2(pb[i >> 2][i & 3], lt);
+      for (int i = 0; i < 8; ++i) {
+        const float x0 = s[2 * i] * c, x1 = s[2 * i + 1] * c;
+        pb[i >> 2][i & 3] = E::pack2(exp2_fast(x0 - m_use), exp2_fast(x1 - m_use));
+        lt = E::sum2(pb[i >> 2][i & 3], lt);
+      }
+    } else {
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        pb[i >> 2][i & 3] = E::pack2(exp2_fast(__builtin_fmaf(s[2 * i], c, -m_use)),
+                                     exp2_fast(__builtin_fmaf(s[2 * i + 1], c, -m_use)));
+        lt = E::sum2(pb[i >> 2][i & 3], lt);
+      }
     }
     l_run += lt;
   };

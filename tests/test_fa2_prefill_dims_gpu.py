@@ -86,3 +86,21 @@ def test_scales_that_are_not_positive(scale, B, T, d):
         *(_lib.strides(t) for t in (q, k, v, o)), None, 1, scale, _lib.stream_of(q)))
     qs = q.float().cpu() * (scale * math.sqrt(d))   # the oracle scales by 1 / sqrt(d)
     check_close(o, sdpa.attention_ref(qs, k.float().cpu(), v.float().cpu(), True), torch.bfloat16, "scale")
+
+
+@DTYPES
+@pytest.mark.parametrize("d", [32, 64, 256])
+@pytest.mark.parametrize("B,T", [(1, 1000), (4, 1000)])
+@pytest.mark.parametrize("size", [2.0 ** 9, 2.0 ** 15])
+def test_scores_past_the_reach_of_the_exponents_fraction(size, B, T, d, dtype):
+    """Scores of 2^20 to 2^38, whose rounding alone is more than an exponent holds: each query's largest
+    one has all the weight."""
+    g = torch.Generator().manual_seed(d)
+    q, k, v = (torch.randn(B, n, T, d, generator=g) for n in (12, 2, 2))
+    q, k, v = (q.sign() * size).to(dtype), (k.sign() * size).to(dtype), v.to(dtype)
+    # scores are whole multiples of size^2: a query's largest stands out by at least 2 of them, or is
+    # shared by keys that weigh the same
+    announce(f"[gpu] prefill dims: scores of {size}^2, {B} x {T} x {d} {dtype}")
+    out = FlashAttention2Function.apply(q.cuda(), k.cuda(), v.cuda(), False, None)
+    torch.cuda.synchronize()
+    check_close(out, sdpa.attention_ref(q, k, v, False), dtype, "large scores")
