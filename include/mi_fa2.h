@@ -77,7 +77,8 @@ MI_FA2_API const char* mi_fa2_last_error(void);
  *   prefill_one_stream_min_work_groups, prefill_one_stream_max_keys: prefill launches of at
  *   least that many work-groups (two per CU) whose query tiles see at most that many keys take
  *   the one-stream work-group shape (4 waves, two work-groups per CU), the others the two-stream
- *   shape (8 waves, one per CU); MI_FA2_PREFILL_STREAMS=1 or 2 forces one shape.
+ *   shape (8 waves, one per CU); MI_FA2_PREFILL_STREAMS=1 or 2 forces one shape, whose launches
+ *   are not split over keys either.
  */
 typedef struct mi_fa2_plan {
   int32_t num_cus;

@@ -20,6 +20,7 @@ hipError_t launch_prefill(const FwdParams& p, int dtype, int mode, int max_seqle
 int prefill_split_pieces(int n_cus, int64_t batch, int heads_q, int heads_kv, int64_t seqlen_q,
                          int64_t max_kv);
 size_t prefill_split_bytes(int64_t batch, int heads_q, int heads_kv, int64_t seqlen_q, int pieces);
+int prefill_forced_streams();
 hipError_t launch_prefill_split(const FwdParams& p, int dtype, int mode, int pieces,
                                 hipStream_t stream);
 hipError_t launch_decode(const FwdParams& p, int dtype, int mode, hipStream_t stream);
@@ -239,13 +240,14 @@ size_t split_workspace(int64_t batch, int heads_q, int heads_kv, int64_t seqlen_
 
 int launched(hipError_t err);
 
-// The padded prefill of p, split if the workspace allows.
+// The padded prefill of p, split if the workspace allows and no shape is forced.
 int run_prefill(FwdParams& p, const Plan& plan, int dtype, int mode, void* workspace,
                 size_t workspace_bytes, hipStream_t s) {
   const int pieces = mi_fa2::prefill_split_pieces(std::min(plan.cus, kSplitCus), p.B, p.Hq, p.Hkv,
                                                   p.T, p.S);
   const size_t need = mi_fa2::prefill_split_bytes(p.B, p.Hq, p.Hkv, p.T, pieces);
-  if (need && workspace && workspace_bytes >= need && aligned16(workspace)) {
+  if (need && workspace && workspace_bytes >= need && aligned16(workspace) &&
+      !mi_fa2::prefill_forced_streams()) {
     p.ws_o = static_cast<float*>(workspace);
     return launched(mi_fa2::launch_prefill_split(p, dtype, mode, pieces, s));
   }

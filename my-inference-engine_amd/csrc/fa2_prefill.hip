@@ -1013,6 +1013,13 @@ hipError_t launch_prefill_split(const FwdParams& p, int dtype, int mode, int pie
                         : launch_prefill_split_t<FP16, kDense>(p, pieces, stream);
 }
 
+// The shape MI_FA2_PREFILL_STREAMS = 1 or 2 forces on every prefill launch, which then is not split
+// either, or 0 (read at every launch, so that a test can run both in one process).
+int prefill_forced_streams() {
+  const char* e = std::getenv("MI_FA2_PREFILL_STREAMS");
+  return e != nullptr && (e[0] == '1' || e[0] == '2') && e[1] == 0 ? e[0] - '0' : 0;
+}
+
 // Key streams per work-group for a launch of `grid` work-groups whose query tiles see at most
 // `max_keys` keys.  Two streams halve the time of the longest query tile, which is what bounds a
 // launch of about one work-group per CU (one long causal sequence); one stream fits two
@@ -1020,11 +1027,9 @@ hipError_t launch_prefill_split(const FwdParams& p, int dtype, int mode, int pie
 // behind the other's key loop once there are enough work-groups to fill both slots of every CU
 // and the tiles are short enough for those to matter.  Measured (us per launch, two streams / one
 // stream): 2 x 4096 causal 111.1 / 107.5, 3 x 4096 165.8 / 159.3, 16 packed rows of up to 1024
-// 40.8 / 30.6; 1 x 6144 causal 122.8 / 134.4, 1 x 16384 causal 726 / 741.  MI_FA2_PREFILL_STREAMS
-// = 1 or 2 forces one shape (read at every launch, so that a test can run both in one process).
+// 40.8 / 30.6; 1 x 6144 causal 122.8 / 134.4, 1 x 16384 causal 726 / 741.
 static int prefill_streams(int grid, int n_cus, int max_keys) {
-  const char* e = std::getenv("MI_FA2_PREFILL_STREAMS");
-  if (e != nullptr && (e[0] == '1' || e[0] == '2') && e[1] == 0) return e[0] - '0';
+  if (const int forced = prefill_forced_streams()) return forced;
   return grid >= prefill_one_stream_min_grid(n_cus) && max_keys <= kPrefillOneStreamMaxKeys ? 1
                                                                                             : 2;
 }

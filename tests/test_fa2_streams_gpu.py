@@ -84,3 +84,17 @@ def test_ragged_varlen_lse(streams):
         want = sdpa.lse_ref(qb, kb, True)[0]
         # bf16-rounded P in the row sum: within log(1 + 2^-8) of the exact LSE
         assert (lse[:, s:e] - want).abs().max().item() < math.log1p(2.0 ** -8) + 1e-4, f"row {b}"
+
+
+def test_a_forced_shape_is_not_split(streams):
+    """Few queries over many keys, which would be cut into pieces: the forced shape runs them whole, so a
+    workspace changes nothing."""
+    from test_fa2_key_split_gpu import unsplit, ws_bytes
+    assert ws_bytes(1, 12, 2, 150, 3001) > 0
+    q, k, v = (t[:, :, :3001].cuda() for t in wl.prefill_single(3001, seed=9))
+    q = q[:, :, -150:].contiguous()
+    k, v = k.contiguous(), v.contiguous()
+    announce(f"[gpu] streams {streams}: 150 queries over 3001 keys, with and without a workspace")
+    out = FlashAttention2Function.apply(q, k, v, True, None)
+    lens = torch.tensor([3001], dtype=torch.int32, device="cuda")
+    assert torch.equal(out, unsplit(q, k, v, True, lens)[0])
