@@ -13,13 +13,12 @@
 #include <utility>
 
 #include "fa2_common.h"
+#include "fa2_split_rule.h"
 
 namespace mi_fa2 {
 hipError_t launch_prefill(const FwdParams& p, int dtype, int mode, int max_seqlen_q,
                           hipStream_t stream);
-int prefill_split_pieces(int n_cus, int64_t batch, int heads_q, int heads_kv, int64_t seqlen_q,
-                         int64_t max_kv);
-size_t prefill_split_bytes(int64_t batch, int heads_q, int heads_kv, int64_t seqlen_q, int pieces);
+size_t prefill_split_bytes(const SplitPlan& plan);
 int prefill_forced_streams();
 hipError_t launch_prefill_split(const FwdParams& p, int dtype, int mode, int pieces,
                                 hipStream_t stream);
@@ -233,9 +232,8 @@ size_t decode_workspace(int64_t batch, int64_t heads_q, int64_t heads_kv, int64_
 // call without it runs unsplit.
 constexpr int kSplitCus = 256;
 size_t split_workspace(int64_t batch, int heads_q, int heads_kv, int64_t seqlen_q, int64_t max_kv) {
-  const int pieces =
-      mi_fa2::prefill_split_pieces(kSplitCus, batch, heads_q, heads_kv, seqlen_q, max_kv);
-  return mi_fa2::prefill_split_bytes(batch, heads_q, heads_kv, seqlen_q, pieces);
+  return mi_fa2::prefill_split_bytes(
+      mi_fa2::split_plan(kSplitCus, batch, heads_q, heads_kv, seqlen_q, max_kv));
 }
 
 int launched(hipError_t err);
@@ -243,13 +241,15 @@ int launched(hipError_t err);
 // The padded prefill of p, split if the workspace allows and no shape is forced.
 int run_prefill(FwdParams& p, const Plan& plan, int dtype, int mode, void* workspace,
                 size_t workspace_bytes, hipStream_t s) {
-  const int pieces = mi_fa2::prefill_split_pieces(std::min(plan.cus, kSplitCus), p.B, p.Hq, p.Hkv,
-                                                  p.T, p.S);
-  const size_t need = mi_fa2::prefill_split_bytes(p.B, p.Hq, p.Hkv, p.T, pieces);
+  const mi_fa2::SplitPlan split =
+      mi_fa2::split_plan(std::min(plan.cus, kSplitCus), p.B, p.Hq, p.Hkv, p.T, p.S,
+                         mode == mi_fa2::kPaged ? std::max(p.block_size, mi_fa2::kSplitStep)
+                                                : mi_fa2::kSplitStep);
+  const size_t need = mi_fa2::prefill_split_bytes(split);
   if (need && workspace && workspace_bytes >= need && aligned16(workspace) &&
       !mi_fa2::prefill_forced_streams()) {
     p.ws_o = static_cast<float*>(workspace);
-    return launched(mi_fa2::launch_prefill_split(p, dtype, mode, pieces, s));
+    return launched(mi_fa2::launch_prefill_split(p, dtype, mode, split.pieces, s));
   }
   return launched(mi_fa2::launch_prefill(p, dtype, mode, p.T, s));
 }

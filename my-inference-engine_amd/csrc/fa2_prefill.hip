@@ -44,6 +44,7 @@
 //     kv head run on the same XCDs (one L2 holds their K/V) and every XCD takes its tiles longest
 //     first, so causal work drains evenly.
 #include "fa2_common.h"
+#include "fa2_split_rule.h"
 #include "fa2_tiles.h"
 
 #include <cstdlib>
@@ -947,44 +948,10 @@ __global__ __launch_bounds__(256) void fa2_prefill_combine_kernel(const FwdParam
         L > 0.f ? (M + __builtin_log2f(L)) * kLn2 : -INFINITY;
 }
 
-static int64_t split_tiles(int64_t batch, int heads_q, int heads_kv, int64_t seqlen_q) {
-  return batch * heads_kv * ((seqlen_q * (heads_q / heads_kv) + kPfRows - 1) / kPfRows);
-}
+static_assert(kSplitRows == kPfRows && kSplitStep == PfShape<2>::kStep, "the rule's sizes");
 
-// Pieces each tile's keys are cut into for a padded launch (1: none) on a device of n_cus CUs, the
-// number with the least time by this model (us, fitted to 18 shapes of 5 to 700 queries over 900 to
-// 8,000 keys at 1 to 63 pieces, within 10% of the best of them everywhere):
-//   unsplit, one work-group per CU or fewer:  6.5 + 1.45 per 128-key step of the longest tile;
-//   split, one work-group per CU or fewer:    9.5 + 1.45 per step of a piece
-//       + 0.033 per tile and piece (its partials written and read) + 0.05 per piece (the merge).
-// Measured unsplit -> split: 150 queries over 3,001 keys 42.4 -> 19.6 us, 5 over 8,000 92.6 -> 13.9,
-// 700 over 4,000 53.9 -> 35.8; 700 over 1,000 stays unsplit (19.1, split 21.8).
-int prefill_split_pieces(int n_cus, int64_t batch, int heads_q, int heads_kv, int64_t seqlen_q,
-                         int64_t max_kv) {
-  const int64_t unsplit = batch * heads_q * ((seqlen_q + kPfRows - 1) / kPfRows);
-  if (seqlen_q < 1 || unsplit < 1 || unsplit > n_cus) return 1;
-  const int64_t tiles = split_tiles(batch, heads_q, heads_kv, seqlen_q);
-  const int64_t row_groups =   // of 32 rows, four to a tile: what is written
-      batch * heads_kv * ((seqlen_q * (heads_q / heads_kv) + 31) / 32);
-  const int64_t steps = (max_kv + PfShape<2>::kStep - 1) / PfShape<2>::kStep;
-  const int64_t most = std::min<int64_t>(n_cus / tiles, steps);
-  int best = 1;
-  int64_t best_cost = 650 + 145 * steps - 100;   // in 10 ns; a split has to gain 1 us
-  for (int64_t s = 2; s <= most; ++s) {
-    const int64_t each = (steps + s - 1) / s;
-    const int64_t cost = 950 + 145 * each + 33 * row_groups * s / 40 + 5 * s;
-    if (cost < best_cost) {
-      best_cost = cost;
-      best = (int)s;
-    }
-  }
-  return best;
-}
-
-size_t prefill_split_bytes(int64_t batch, int heads_q, int heads_kv, int64_t seqlen_q, int pieces) {
-  return pieces > 1 ? (size_t)split_tiles(batch, heads_q, heads_kv, seqlen_q) * pieces *
-                          kPartFloats * sizeof(float)
-                    : 0;
+size_t prefill_split_bytes(const SplitPlan& plan) {
+  return plan.pieces > 1 ? (size_t)plan.tiles * plan.pieces * kPartFloats * sizeof(float) : 0;
 }
 
 // The split launch of p (padded modes): p.ws_o holds prefill_split_bytes.
