@@ -327,7 +327,9 @@ def fa2_paged(q, k_pool, v_pool, block_table, kv_lens, *, block_size=16, max_kv_
     block_table  [B, W] int32: row b's token p is at slot block_table[b, p // block_size] *
                  block_size + p % block_size (kv_cache.py:15-16)
     kv_lens      [B] int32: keys per row including this step's T (model.py:175)
-    max_kv_len   host-side upper bound of kv_lens (default W * block_size)
+    max_kv_len   host-side upper bound of kv_lens (default W * block_size); the longest row's length,
+                 where it is known: few queries over many keys are split over work-groups by it, and
+                 not at all by the default, which says nothing of the lengths
     is_causal    default T > 1, as model.py:185 sets it; bottom-right aligned per row
     out          optional [B, Hq, T, 128] output (any row/head/token strides, 16-byte aligned)
     Returns O [B, Hq, T, 128] (and the fp32 LSE [B, Hq, T] if return_lse).
@@ -399,6 +401,11 @@ def _plan_paged(q, k_pool, v_pool, block_table, kv_lens, block_size, max_kv_len,
     assert block_size >= 16 and block_size & (block_size - 1) == 0, "block_size: power of 2, >= 16"
     assert k_pool.shape[0] % block_size == 0, "pool slots must be whole blocks"
     _envelope(q, k_pool, v_pool)
+    decodes = _decodes(T, Hq // Hkv, B)
+    # Splitting a prefill by a bound far above the true lengths costs more than it gives (150 queries
+    # over 150 keys of a capacity of 8,192: 9.2 us whole, 16.5 in pieces; over all 8,192: 101 and 27), so
+    # it takes one that the caller has given.  (The decode's workspace is not a choice.)
+    wants_ws = decodes or max_kv_len is not None
     if max_kv_len is None:
         max_kv_len = block_table.shape[1] * block_size
     # kv_lens are clamped to max_kv_len in-kernel, so this bound keeps every table read in range
@@ -416,8 +423,8 @@ def _plan_paged(q, k_pool, v_pool, block_table, kv_lens, block_size, max_kv_len,
             _strides_of(q.shape[:3], _contig(q.shape[:3])) if return_lse else None,
             (B, Hq, Hkv, T, max_kv_len, d, block_size, k_pool.shape[0] // block_size),
             (int(bool(is_causal)), 1.0 / math.sqrt(d)),
-            _workspace if _decodes(T, Hq // Hkv, B) else _own_workspace,
-            _paged_ws_bytes(B, Hq, Hkv, T, max_kv_len, d))
+            _workspace if decodes else _own_workspace,
+            _paged_ws_bytes(B, Hq, Hkv, T, max_kv_len, d) if wants_ws else 0)
 
 
 _WS_BYTES = {}

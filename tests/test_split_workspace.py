@@ -27,11 +27,11 @@ def padded(T, group):
     return lambda: fa2.FlashAttention2Function.apply(q, k, k, T > 1, None)
 
 
-def paged(T, group):
+def paged(T, group, max_kv_len=4096):
     q, pool = on_gpu(1, 2 * group, T, 128), on_gpu(4096, 2, 128)
     table = torch.arange(256, dtype=torch.int32)[None]
     lens = torch.tensor([4096], dtype=torch.int32)
-    return lambda: fa2.fa2_paged(q, pool, pool, table, lens)
+    return lambda: fa2.fa2_paged(q, pool, pool, table, lens, max_kv_len=max_kv_len)
 
 
 @pytest.mark.parametrize("T,group", [(150, 6), (2, 1), (1, 17)])
@@ -62,6 +62,26 @@ def test_calls_that_overlap_have_their_own_partials(call, entry, T, group, monke
     (a, n), (b, m) = seen
     assert n == m > 0 and a and b
     assert a + n <= b or b + m <= a
+
+
+def test_paged_prefills_are_split_by_a_bound_that_was_given(monkeypatch):
+    """Without one the table's capacity bounds the lengths, which may be far shorter."""
+    lib, seen = _lib.load(), []
+
+    class Lib:
+        def __getattr__(self, name):
+            return (lambda *a: seen.append(a[-3]) or 0) if name == "mi_fa2_fwd_paged" else getattr(lib, name)
+
+    monkeypatch.setattr(_lib, "load", lambda: Lib())
+    monkeypatch.setattr(_lib, "on_device", lambda dev: contextlib.nullcontext(0))
+    monkeypatch.setattr(_lib, "device_index", lambda dev: 0)
+    monkeypatch.setattr(torch._C, "_cuda_getCurrentRawStream", lambda i: 0, raising=False)
+    for bound in (4096, None, 4096):   # each time by its own plan
+        paged(150, 6, bound)()
+    assert [ws is not None for ws in seen] == [True, False, True]
+    seen.clear()
+    paged(1, 6, None)()   # the decode needs its workspace
+    assert seen[0] is not None
 
 
 def test_a_call_without_memory_for_partials_runs_unsplit(monkeypatch):
