@@ -88,14 +88,16 @@ def _readable(t):
 def _held(t, x):
     """Whether parameter t is held as the kernels read it for rows like x: x's type and device,
     contiguous, 16-byte aligned, a plain tensor (no subclass with operations of its own)."""
-    return (type(t) in _PLAIN and t.dtype == x.dtype and t.device == x.device and t.is_contiguous()
-            and t.data_ptr() % 16 == 0)
+    return (type(t) in _PLAIN and t.dtype == x.dtype and t.get_device() == x.get_device()
+            and t.is_contiguous() and t.data_ptr() % 16 == 0)
 
 
 def weight_fits(w, x, out_features):
     """Whether w is an [out_features, in] weight the kernel reads for rows like x."""
-    return (_held(w, x) and w.dim() == 2 and w.shape[0] == out_features and out_features % 16 == 0
-            and out_features > 0 and w.shape[1] % 32 == 0 and 0 < w.shape[1] <= MAX_IN)
+    if not _held(w, x) or w.dim() != 2:
+        return False
+    n, k = w.shape
+    return n == out_features and n % 16 == 0 and n > 0 and k % 32 == 0 and 0 < k <= MAX_IN
 
 
 def bias_fits(b, x, out_features):
@@ -107,17 +109,18 @@ def linear_fits(x, w, norm=None):
     """Whether `linear` takes x [rows, in] and w [out, in] (and norm, an RMSNorm weight)."""
     if norm is not None and not (_held(norm, x) and norm.shape == x.shape[1:]):
         return False
-    return (type(x) in _PLAIN and 1 <= x.shape[0] <= (MAX_ROWS if norm is None else MAX_NORM_ROWS)
+    rows, k = x.shape
+    return (type(x) in _PLAIN and 1 <= rows <= (MAX_ROWS if norm is None else MAX_NORM_ROWS)
             and x.dtype in _lib.DTYPES and weight_fits(w, x, w.shape[0])
-            and w.shape[1] == x.shape[1] and _readable(x))
+            and w.shape[1] == k and _readable(x))
 
 
 def mlp_fits(x, gate_up_w, down_w, norm=None):
     """Whether `mlp` takes x [rows, hidden] and these weights (and norm, an RMSNorm weight)."""
-    hidden, inter = x.shape[1], down_w.shape[1]
-    return (linear_fits(x, gate_up_w, norm) and hidden % 16 == 0 and inter % 32 == 0
-            and 0 < inter <= 1 << 18 and gate_up_w.shape[0] == 2 * inter
-            and down_w.shape[0] == hidden and _held(down_w, x))
+    hidden, inter = down_w.shape
+    return (linear_fits(x, gate_up_w, norm) and x.shape[1] == hidden and hidden % 16 == 0
+            and inter % 32 == 0 and 0 < inter <= 1 << 18 and gate_up_w.shape[0] == 2 * inter
+            and _held(down_w, x))
 
 
 def linear(x, w, bias=None, residual=None, norm_weight=None, eps=0.0, out=None):

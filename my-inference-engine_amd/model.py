@@ -101,11 +101,14 @@ def transposed(weight):
 def plain(*modules):
     """Whether the modules are exactly these classes with nothing hooked on and no forward of their
     own, so that a kernel may do their work without calling them."""
-    return (not nn.modules.module._has_any_global_hook()
-            and all(type(m) in (nn.Linear, RMSNorm, Attention, MLP, Block)
-                    and "forward" not in vars(m)
-                    and not (m._forward_hooks or m._forward_pre_hooks or m._backward_hooks
-                             or m._backward_pre_hooks) for m in modules))
+    if nn.modules.module._has_any_global_hook():
+        return False
+    for m in modules:
+        d = vars(m)
+        if (type(m) not in _PLAIN or "forward" in d or d["_forward_hooks"] or d["_forward_pre_hooks"]
+                or d["_backward_hooks"] or d["_backward_pre_hooks"]):
+            return False
+    return True
 
 
 def inference(*tensors):
@@ -268,10 +271,11 @@ class MLP(nn.Module):
     def few_rows_fit(self, x, norm=None):
         """Whether few_rows.mlp does this module's work on x [tokens, hidden] (after `norm`)."""
         gu, down = self.gate_up_proj, self.down_proj
-        return (plain(gu, down, *((self, norm) if norm is not None else ()))
-                and gu.bias is None and down.bias is None and inference(x, gu.weight, down.weight)
-                and few_rows.mlp_fits(x, gu.weight, down.weight,
-                                      norm.weight if norm is not None else None))
+        if not plain(gu, down, *((self, norm) if norm is not None else ())):
+            return False
+        gw, dw = gu.weight, down.weight
+        return (gu.bias is None and down.bias is None and inference(x, gw, dw)
+                and few_rows.mlp_fits(x, gw, dw, norm.weight if norm is not None else None))
 
 
 class Block(nn.Module):
@@ -285,6 +289,9 @@ class Block(nn.Module):
     def forward(self, x, cos, sin, cache, layer, meta):
         x = x + self.self_attn(self.input_layernorm(x), cos, sin, cache, layer, meta)
         return x + self.mlp(self.post_attention_layernorm(x))
+
+
+_PLAIN = (nn.Linear, RMSNorm, Attention, MLP, Block)   # what plain() knows
 
 
 class Qwen2ForCausalLM(nn.Module):
