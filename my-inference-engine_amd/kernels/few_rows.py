@@ -123,6 +123,23 @@ def mlp_fits(x, gate_up_w, down_w, norm=None):
             and _held(down_w, x))
 
 
+def linear_pays(rows, w):
+    """Whether `linear` on [rows, in] is at least as fast as the library's GEMM (us, library and here, bf16;
+    fp16 alike).  Up to 16 rows: from 768 in features on (896 x 32,000 14.6 and 13.5, 2,048 x 151,936
+    150 and 122; 512 x 32,000 10.5 and 12.1).  More rows: where the weight is larger than the 256 MB
+    last-level cache, whose stream bounds both (1,536 x 151,936 at 17, 32, 40 rows 103 and 90, 105 and
+    96, 106 and 100; 1,536 x 64,000 at 32 33.8 and 35.3), up to 40 rows (48: 98 and 102)."""
+    return (rows <= 16 and w.shape[1] >= 768) or (
+        rows <= 40 and w.numel() * w.element_size() >= 1 << 28)
+
+
+def mlp_pays(rows, hidden):
+    """The same for `mlp`: up to 32 rows, and up to 64 where hidden <= 1536 (1,536 x 8,960 at 16, 32, 64
+    rows 41 and 24, 41 and 29, 48 and 37; 1,792 x 4,864 at 32 and 33 24.8 and 22.5, 26.0 and 28.0;
+    2,048 x 8,192 at 33 35.2 and 38.2)."""
+    return rows <= (MAX_ROWS if hidden <= 1536 else 32)
+
+
 def linear(x, w, bias=None, residual=None, norm_weight=None, eps=0.0, out=None):
     """x [rows, in], w [out, in] -> [rows, out].  residual [rows, out] may be `out` (in place)."""
     R, K = x.shape

@@ -258,7 +258,7 @@ class MLP(nn.Module):
     def forward(self, x):
         if x.is_cuda:
             rows = x.reshape(-1, x.shape[-1])
-            if rows.shape[0] <= few_rows.MAX_ROWS and self.few_rows_fit(rows):
+            if few_rows.mlp_pays(*rows.shape) and self.few_rows_fit(rows):
                 return few_rows.mlp(rows, self.gate_up_proj.weight,
                                     self.down_proj.weight).view(x.shape)
             gu = rows @ transposed(self.gate_up_proj.weight)
@@ -364,7 +364,7 @@ class Qwen2ForCausalLM(nn.Module):
         w = self.embed_tokens.weight
         if x.is_cuda:
             rows = x.reshape(-1, x.shape[-1])
-            if (rows.shape[0] <= few_rows.MAX_ROWS and inference(x, w)
+            if (few_rows.linear_pays(rows.shape[0], w) and inference(x, w)
                     and few_rows.linear_fits(rows, w)):
                 return few_rows.linear(rows, w).view(*x.shape[:-1], w.shape[0])
             return x @ transposed(w)

@@ -3,6 +3,7 @@ import pytest
 import torch
 
 from conftest import announce
+from kernels import few_rows
 from kv_cache import KVCache
 from model import QwenConfig, Qwen2ForCausalLM
 
@@ -11,9 +12,9 @@ CFG = QwenConfig(hidden_size=256, num_layers=2, num_heads=2, num_kv_heads=1, int
                  vocab_size=512)
 
 
-def make(cls=Qwen2ForCausalLM, dtype=torch.bfloat16):
-    model = cls(CFG).cuda().init_random(std=0.05, seed=0).to(dtype).eval().requires_grad_(False)
-    return model
+def make(cfg=CFG):
+    return (Qwen2ForCausalLM(cfg).cuda().init_random(std=0.05, seed=0).to(torch.bfloat16).eval()
+            .requires_grad_(False))
 
 
 def decode(model, steps=3, rows=3):
@@ -130,19 +131,24 @@ def test_watched_layers_are_called(how):
     close(got, plain)
 
 
-def test_the_head_follows_torch_where_torch_is_followed():
+def test_the_head_follows_torch_where_torch_is_followed(monkeypatch):
     """Forward mode, vmap, a dispatch mode and autocast see the head's product as they would any other."""
     from torch.utils.flop_counter import FlopCounterMode
-    model = make()
+    H, V = 768, 512
+    model = make(cfg=QwenConfig(hidden_size=H, num_layers=1, num_heads=2, num_kv_heads=1,
+                                intermediate_size=512, vocab_size=V))
     w = model.embed_tokens.weight
-    x, t = (torch.randn(4, 1, CFG.hidden_size, dtype=torch.bfloat16, device="cuda") for _ in range(2))
+    x, t = (torch.randn(4, 1, H, dtype=torch.bfloat16, device="cuda") for _ in range(2))
+    fused, linear = [], few_rows.linear
+    monkeypatch.setattr(few_rows, "linear", lambda *a, **k: fused.append(1) or linear(*a, **k))
     announce("[gpu] head under forward mode, vmap, a dispatch mode and autocast")
     with torch.no_grad():
         want = model.lm_head(x)
+        assert len(fused) == 1
         close(torch.func.vmap(model.lm_head)(x), want)
         with FlopCounterMode(display=False) as flops:
             close(model.lm_head(x), want)
-        assert flops.get_total_flops() == 2 * 4 * CFG.hidden_size * CFG.vocab_size
+        assert flops.get_total_flops() == 2 * 4 * H * V
         with torch.autograd.forward_ad.dual_level():
             y = model.lm_head(torch.autograd.forward_ad.make_dual(x, t))
             tangent = torch.autograd.forward_ad.unpack_dual(y).tangent
@@ -153,3 +159,4 @@ def test_the_head_follows_torch_where_torch_is_followed():
     grad = x.clone().requires_grad_(True)
     model.lm_head(grad).sum().backward()
     assert grad.grad is not None
+    assert len(fused) == 1   # none of these
