@@ -361,8 +361,14 @@ __global__ __launch_bounds__(64 * kGenWaves) void fa2_general_kernel(FwdParams p
 // to each work-group (d_v <= 128).  Bound by the latency of a pair's loads and, where two
 // work-groups share a CU, by the longer one's chain: wide V loads and pairing long with short tiles
 // took 1 x 12 x 512 x 128 fp32 from 36.0 to 25.9 us, 1 x 12 x 1000 x 256 bf16 from 142 to 87.
+// Two waves per SIMD, so that two work-groups of four share a CU, where their registers allow without
+// spilling.
+template <class E, int D, int DV>
+constexpr int kSplitOcc =
+    DV == 256 && (D == 256 || (D >= 64 && sizeof(typename Gen<E>::T) == 4)) ? 1 : 2;
+
 template <class E, int D, int DV, int W, bool AHEAD>
-__global__ __launch_bounds__(64 * W) void fa2_general_split_kernel(FwdParams p) {
+__global__ __launch_bounds__(64 * W, (kSplitOcc<E, D, DV>)) void fa2_general_split_kernel(FwdParams p) {
   constexpr int kGenWaves = W;
   using G = Gen<E>;
   using T = typename G::T;
