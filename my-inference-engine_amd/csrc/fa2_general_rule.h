@@ -47,7 +47,10 @@ inline GeneralKernel general_kernel(const GeneralCall& c) {
   //  * instead of the split kernel (d <= 64; at d = 256 it is the closer one to 64 bits), where its
   //    shape of 64 rows gains: by the work, 16-row tiles x keys.  d = 64, split and 64-row: 2 x 300
   //    (137 K) 8.7 and 9.0, 4 x 200 (125 K) 8.1 and 7.8, 3 x 300 (205 K) 10.3 and 9.2, 1 x 700
-  //    (370 K) 14.2 and 11.0, 1 x 1000 (756 K) 19.2 and 13.5; d = 32 the same within 0.3;
+  //    (370 K) 14.2 and 11.0, 1 x 1000 (756 K) 19.2 and 13.5; d = 32 the same within 0.3; and with more
+  //    of those tiles than CUs: up to there the split kernel has a CU and eight waves for each (1 x 300
+  //    over 4,000 keys, 228 tiles, d = 64 26.8 and 36.6, d = 32 19.5 and 27.4; 1 x 400 over 2,000, 300
+  //    tiles, 25.1 and 22.0, 18.5 and 16.3);
   //  * instead of the staged kernel, from one full tile of queries on: d = 64, 4 x 64 4.8 staged and
   //    6.3, 4 x 200 9.0 and 8.3, 4 x 1000 36.7 and 20.9.
   // Of its two shapes, the 64-row one while its work-groups run at once (d = 32: two per CU) and, where
@@ -56,7 +59,8 @@ inline GeneralKernel general_kernel(const GeneralCall& c) {
   // d = 32, 4 x 512 8.6 and 9.2, 4 x 1000 15.9 and 15.3.
   if (c.bits16 && c.d == c.dv && (c.d == 32 || c.d == 64 || c.d == 256)) {
     const int64_t tiles16 = (c.seqlen_q + kRows - 1) / kRows * heads;
-    const bool better = split ? c.d <= 64 && c.seqlen_q >= kRows && tiles16 * c.seqlen_k >= 150000
+    const bool better = split ? c.d <= 64 && c.seqlen_q >= kRows && tiles16 > c.n_cus &&
+                                    tiles16 * c.seqlen_k >= 150000
                               : c.seqlen_q >= 128;
     const bool small = c.d == 32   ? tiles <= 2 * c.n_cus
                        : c.d == 64 ? 4 * tiles <= 3 * c.n_cus ||

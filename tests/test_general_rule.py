@@ -12,6 +12,11 @@ def test_the_kernels_and_their_sizes():
     assert kernel(4, 12, 2, 1000, 1000, 256) == DIMS
     assert kernel(32, 12, 2, 64, 64, 64) == kernel(16, 12, 2, 1000, 1000, 16) == STAGED
     assert kernel(1, 12, 2, 200, 200, 64) == kernel(1, 12, 2, 1000, 1000, 256) == SPLIT
+    # few queries over many keys: up to a 16-row tile per CU, each has one to itself on the split kernel
+    for d in (32, 64):
+        assert kernel(1, 12, 2, 300, 8000, d) == kernel(4, 12, 2, 64, 8000, d) == SPLIT
+        assert kernel(64, 12, 2, 1, 500, d) == kernel(64, 12, 2, 15, 500, d) == SPLIT
+        assert kernel(1, 12, 2, 400, 2000, d) == DIMS_SMALL
     assert kernel(4, 12, 2, 1000, 1000, 64, 128) == STAGED
     for d, dv, T in itertools.product((16, 32, 64, 128, 256), (16, 32, 64, 128, 256), (1, 64, 4096)):
         assert kernel(16, 12, 2, T, T, d, dv, bits16=False) == SPLIT
