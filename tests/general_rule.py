@@ -29,3 +29,10 @@ def kernel(B, Hq, Hkv, T, S, d, dv=None, bits16=True, scale=0.1, strides=None, n
     dv = d if dv is None else dv
     sizes = (ctypes.c_int64 * 7)(B, Hq, Hkv, T, S, *(strides or (d, dv)))
     return _library()(sizes, d, dv, bits16, scale, n_cus, xcd_log2)
+
+
+def on_this_device(*sizes, **kw):
+    """The kernel a call of these sizes takes on the current GPU."""
+    from kernels import _lib
+    plan = _lib.launch_plan()
+    return kernel(*sizes, **kw, n_cus=plan["num_cus"], xcd_log2=plan["xcds_mapped"].bit_length() - 1)

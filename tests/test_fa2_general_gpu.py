@@ -21,6 +21,7 @@ import torch
 from conftest import announce
 from kernels.fa2 import FlashAttention2Function, fa2_forward
 from oracle import sdpa
+import general_rule as rule
 import workloads as wl
 
 pytestmark = pytest.mark.gpu
@@ -183,19 +184,25 @@ def test_long_rows_and_single_queries(dtype):
 @pytest.mark.parametrize("causal", [True, False], ids=["causal", "full"])
 def test_both_work_splits(dtype, causal):
     """The launcher picks the LDS-staged kernel (64 query rows per work-group, K/V shared by its 4
-    waves) when there are at least 64 query rows and 256 such work-groups, else the key-split one
-    (16 rows per work-group, keys split over its 4 waves): shapes on both sides of that line."""
+    waves) for 16-bit calls of at least 64 query rows and 256 such work-groups, else, and for fp32, the
+    key-split one (16 rows per work-group, keys split over its 4 or 8 waves); equal head dims of 32, 64
+    and 256 leave both for the prefill kernel where they are larger: shapes on both sides of those
+    lines, fp32 on the key-split kernel in every one."""
     g = torch.Generator().manual_seed(9)
-    for B, Hq, Hkv, T, S, d, d_v in ((4, 16, 4, 256, 300, 64, 64),     # 4*16*4 = 256: LDS-staged
-                                     (4, 16, 4, 256, 300, 32, 128),
-                                     (4, 15, 5, 256, 300, 64, 64),      # 4*15*4 = 240: key-split
-                                     (2, 8, 2, 63, 500, 128, 32)):      # 63 rows: key-split
+    for B, Hq, Hkv, T, S, d, d_v, which in ((8, 16, 4, 100, 300, 64, 64, rule.STAGED),    # 8*16*2 = 256
+                                            (4, 16, 4, 256, 300, 32, 128, rule.STAGED),
+                                            (7, 16, 4, 100, 200, 64, 64, rule.DIMS),      # 224, long enough
+                                            (4, 15, 5, 60, 300, 64, 64, rule.SPLIT),
+                                            (4, 16, 4, 256, 300, 64, 64, rule.DIMS),
+                                            (2, 8, 2, 63, 500, 128, 32, rule.SPLIT)):
+        assert rule.on_this_device(B, Hq, Hkv, T, S, d, d_v, bits16=dtype != torch.float32) == (
+            which if dtype != torch.float32 else rule.SPLIT)
         if dtype != torch.float32 and d == d_v == 128:
             continue
         q = rand((B, Hq, T, d), g, dtype)
         k = rand((B, Hkv, S, d), g, dtype)
         v = rand((B, Hkv, S, d_v), g, dtype)
-        lens = [S, S - 37, T, 200][:B]
+        lens = ([S, S - 37, T, 200] * 2)[:B]
         announce(f"[gpu] general: B={B} Hq={Hq} T={T} S={S} d={d} d_v={d_v} {dtype} causal={causal}")
         out, lse = fa2_forward(q.to(DEV), k.to(DEV), v.to(DEV), causal,
                                torch.tensor(lens, dtype=torch.int32, device=DEV), return_lse=True)
@@ -226,18 +233,19 @@ ALL_DIMS = (16, 32, 64, 128, 256)
 @pytest.mark.parametrize("d", ALL_DIMS, ids=[f"d{x}" for x in ALL_DIMS])
 @pytest.mark.parametrize("dtype", DTYPES, ids=IDS)
 def test_staged_kernel_every_head_dim_pair(dtype, d):
-    """Every (d, d_v) pair on the LDS-staged general kernel (64 query rows per work-group, K/V
-    staged in LDS): B=4, Hq=16, T=256 is 256 such work-groups, which reaches it on MI355X's 256
-    CUs.  Covers its 16-bit d=16 path (16x16x16 scores), the 16-bit and fp32 instantiations
-    without the register prefetch ((d + d_v) x element size > 512 bytes, e.g. bf16 256/256 and
-    fp32 256/256 with about 130 KB of LDS), and d_v = 256; causal and not, ragged rows."""
-    from kernels import _lib
-    assert 4 * 16 * 4 >= _lib.launch_plan()["num_cus"], "shape must reach the staged kernel"
-    B, Hq, Hkv, T, S = 4, 16, 4, 256, 300
-    lens = [300, 263, 256, 200]
+    """Every (d, d_v) pair of the 16-bit types on the LDS-staged general kernel (64 query rows per
+    work-group, K/V staged in LDS): B=8, Hq=16, T=100 is 256 work-groups, which reaches it on MI355X's
+    256 CUs, and too few rows for the prefill kernel of the equal pairs.  Covers its d=16 path
+    (16x16x16 scores), the instantiation without the register prefetch (256/256) and d_v = 256; causal
+    and not, ragged rows.  fp32 runs the same shapes on the key-split kernel, four waves to a
+    work-group."""
+    B, Hq, Hkv, T, S = 8, 16, 4, 100, 300
+    lens = [300, 263, 100, 37] * 2
     for d_v in ALL_DIMS:
         if dtype != torch.float32 and d == d_v == 128:
             continue  # the MFMA prefill kernel's shape, covered by tests/test_fa2_gpu.py
+        assert rule.on_this_device(B, Hq, Hkv, T, S, d, d_v, bits16=dtype != torch.float32) == (
+            rule.STAGED if dtype != torch.float32 else rule.SPLIT)
         g = torch.Generator().manual_seed(d * 1000 + d_v)
         q = rand((B, Hq, T, d), g, dtype)
         k = rand((B, Hkv, S, d), g, dtype)
@@ -258,3 +266,25 @@ def test_staged_kernel_every_head_dim_pair(dtype, d):
             assert torch.equal(fin, torch.isfinite(lse.cpu()))
             bar = 1e-4 if dtype == torch.float32 else math.log1p(2.0 ** -8) + 1e-3
             assert (lse.cpu()[fin] - want[fin]).abs().max().item() < bar
+
+
+@pytest.mark.parametrize("T", [40, 200], ids=["eight_waves", "four_waves"])
+@pytest.mark.parametrize("S", [767, 768, 1500])
+@pytest.mark.parametrize("causal", [True, False], ids=["causal", "full"])
+def test_fp32_head_dim_128_with_and_without_the_next_keys_ahead(causal, S, T):
+    """fp32 at d = 128 loads the next keys ahead from 768 keys on; 72 and 312 tiles of 16 rows, on either
+    side of the device's CUs, take the key-split kernel's two shapes."""
+    from kernels import _lib
+    assert (-(-T // 16) * 24 <= _lib.launch_plan()["num_cus"]) == (T == 40)
+    g = torch.Generator().manual_seed(S + T)
+    q = rand((2, 12, T, 128), g, torch.float32)
+    k, v = rand((2, 2, S, 128), g, torch.float32), rand((2, 2, S, 128), g, torch.float32)
+    lens = [S, S - 333]
+    for b, n in enumerate(lens):
+        k[b, :, n:] = PAD_VALUE
+        v[b, :, n:] = PAD_VALUE
+    announce(f"[gpu] general fp32 d=128: T={T} S={S} causal={causal}")
+    out = FlashAttention2Function.apply(q.to(DEV), k.to(DEV), v.to(DEV), causal,
+                                        torch.tensor(lens, dtype=torch.int32, device=DEV))
+    torch.cuda.synchronize()
+    check_close(out, sdpa.attention_ref(q, k, v, causal, lens), torch.float32, f"T={T} S={S}")

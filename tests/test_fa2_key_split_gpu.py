@@ -47,14 +47,15 @@ def check(got, got_lse, want, want_lse, ref):
     assert err.max().item() < 1e-2 and err.mean().item() < 1e-3, err.max().item()
 
 
-# queries: two, a ragged last tile, exactly one tile of packed rows, several tiles; keys: a few steps,
-# a ragged last one, rows shorter than the batch's longest, than their queries, and empty
+# queries: one, of more heads per kv head than the decode takes, two, a ragged last tile, exactly one
+# tile of packed rows, several tiles; keys: a few steps, a ragged last one, rows shorter than the
+# batch's longest, than their queries, and empty
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "fp16"])
 @pytest.mark.parametrize("causal", [True, False])
 @pytest.mark.parametrize("T,heads,lens", [
     (2, (12, 2), [3001]), (150, (12, 2), [3001]), (64, (4, 2), [1153, 40, 0]),
     (128, (1, 1), [8000]), (700, (2, 2), [2048]), (37, (8, 8), [5000, 4999]),
-    (33, (17, 1), [1200])])
+    (33, (17, 1), [1200]), (1, (17, 1), [3001]), (1, (40, 2), [2500, 130, 0])])
 def test_padded(T, heads, lens, causal, dtype):
     Hq, Hkv = heads
     B, S = len(lens), max(lens)

@@ -9,6 +9,7 @@ import torch
 from conftest import announce
 from kernels import _lib
 from kernels.fa2 import FlashAttention2Function, fa2_forward
+from general_rule import DIMS, DIMS_SMALL, on_this_device
 from oracle import sdpa
 from test_fa2_general_gpu import check_close, rand
 
@@ -17,19 +18,26 @@ DTYPES = pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=[
 
 
 # T, S, heads, kv_lens: a last tile of one row, of 127 and of 128; keys one past, one short of and at a
-# tile; rows with fewer keys than queries, one key and none; more heads than XCDs, one kv head; both
-# shapes (64 and 128 rows per work-group)
+# tile; rows with fewer keys than queries, one key and none; more heads than XCDs, one kv head; one step
+# of keys and many.  128-row work-groups at d = 64 and 256; at d = 32 64-row ones but for two shapes.
+SHAPES = [(257, 257, (12, 2), [257, 256, 1, 0, 129]), (383, 383, (12, 6), [383, 300, 129, 65]),
+          (384, 640, (20, 1), [640, 641 - 257, 100]), (130, 320, (16, 2), [320, 319, 64, 63] * 2),
+          (200, 100, (12, 2), [100] * 16), (1025, 1100, (12, 2), [1100, 900]),
+          (513, 513, (12, 4), [513, 512, 449, 100]), (1000, 1000, (12, 2), [1000, 999, 513, 100])]
+# 64-row work-groups (d <= 64)
+SMALL = [(1000, 1000, (12, 2), [1000]), (700, 1300, (6, 6), [1300, 1]), (513, 2000, (12, 1), [1025])]
+CASES = ([(d, *shape, DIMS_SMALL if d == 32 and shape[0] not in (200, 1000) else DIMS)
+          for d in (32, 64, 256) for shape in SHAPES]
+         + [(d, *shape, DIMS_SMALL) for d in (32, 64) for shape in SMALL])
+
+
 @DTYPES
 @pytest.mark.parametrize("causal", [True, False], ids=["causal", "full"])
-@pytest.mark.parametrize("d", [32, 64, 256])
-@pytest.mark.parametrize("T,S,heads,lens", [
-    (257, 257, (12, 2), [257, 256, 1, 0]), (383, 383, (6, 6), [383, 300, 129, 65]),
-    (384, 640, (20, 1), [640, 641 - 257]), (130, 320, (16, 2), [320, 319, 64, 63] * 2),
-    (200, 100, (12, 2), [100] * 16), (1025, 1100, (12, 2), [1100]),
-    (513, 513, (12, 4), [513, 512, 449, 100])])
-def test_against_the_oracle(T, S, heads, lens, d, causal, dtype):
+@pytest.mark.parametrize("d,T,S,heads,lens,which", CASES)
+def test_against_the_oracle(d, T, S, heads, lens, which, causal, dtype):
     Hq, Hkv = heads
     B = len(lens)
+    assert on_this_device(B, Hq, Hkv, T, S, d) == which
     g = torch.Generator().manual_seed(T + S + d)
     q = torch.randn(B, T, Hq, d, generator=g).to(dtype).transpose(1, 2)   # strided heads
     k, v = rand((B, Hkv, S, d), g, dtype), rand((B, Hkv, S, d), g, dtype)
@@ -49,10 +57,13 @@ def test_against_the_oracle(T, S, heads, lens, d, causal, dtype):
 
 
 def test_large_scores_move_the_running_maximum():
-    # each key's score outgrows the one before by far more than the reference may lag (2^8)
+    # every key's score is 8 above the one before (11.5 in the exponent; past 256, where bf16 holds even
+    # numbers, every second one's is 16 above): each tile moves the maximum, and
+    # what earlier tiles summed is scaled away
+    assert on_this_device(4, 12, 2, 300, 300, 64) == DIMS
     g = torch.Generator().manual_seed(3)
     q = torch.ones(4, 12, 300, 64).bfloat16()
-    k = (torch.arange(300).view(1, 1, 300, 1) * torch.ones(4, 2, 300, 64) * 0.25).bfloat16()
+    k = (torch.arange(300).view(1, 1, 300, 1) * torch.ones(4, 2, 300, 64)).bfloat16()
     v = rand((4, 2, 300, 64), g, torch.bfloat16)
     out = FlashAttention2Function.apply(q.cuda(), k.cuda(), v.cuda(), True, None)
     # every output is about one V value, so its rounding to bf16 is not small beside the bars: half a

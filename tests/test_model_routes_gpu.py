@@ -121,6 +121,8 @@ def test_watched_layers_are_called(how):
     model = make()
     x = torch.zeros(3, CFG.hidden_size, dtype=torch.bfloat16, device="cuda")
     assert model._few_rows_fit(x) and model.layers[0].mlp.few_rows_fit(x)
+    with torch.autocast("cuda", torch.float16):
+        assert not model._few_rows_fit(x) and not model.layers[0].mlp.few_rows_fit(x)
     plain = decode(model)
     calls = watch(model, how)
     assert not model._few_rows_fit(x)
