@@ -614,14 +614,12 @@ hipError_t launch_general_t(const FwdParams& p, int dtype, hipStream_t stream) {
   if (kernel == kGenDims || kernel == kGenDimsSmall)
     return launch_prefill_dims(p, dtype, D, kernel == kGenDimsSmall, stream);
   if (kernel == kGenSplit) {
-    // The next pair's K ahead: where two pairs' fit the registers; for fp32 at d = 128, whose waves
-    // then have the whole register file, only on chains long enough to gain by it (1 x 512 26.5 us
-    // without, 34.0 with; 1 x 800 54.4 and 48.8; 1 x 1500 145.7 and 131.9; d = 64, 1 x 512 15.9 and 13.9;
-    // bf16 d = 256, 1 x 1000 83.4 and 64.6).
+    // The next pair's K ahead: where two pairs' fit the registers, and for fp32 at d = 128 only beside
+    // d_v = 256, whose waves have a SIMD to themselves (without and with, us: d_v = 256, 1 x 800 77.7 and
+    // 68.9, 4 x 1000 388 and 340; d_v = 128, 1 x 512 23.9 and 25.5, 4 x 1000 196 and 205; d_v = 16, 1 x 1500
+    // 77.7 and 103; d = d_v = 64, 1 x 512 15.9 and 13.9; bf16 d = 256, 1 x 1000 83.4 and 64.6).
     constexpr int kRowBytes = D * (int)sizeof(typename Gen<E>::T);
-    if constexpr (kRowBytes < 512 || k16) return launch_split_t<E, D, DV, true>(p, stream);
-    else if (kRowBytes == 512 && p.S >= 768) return launch_split_t<E, D, DV, kRowBytes == 512>(p, stream);
-    else return launch_split_t<E, D, DV, false>(p, stream);
+    return launch_split_t<E, D, DV, kRowBytes < 512 || k16 || (kRowBytes == 512 && DV == 256)>(p, stream);
   }
   if constexpr (k16) {
     constexpr int kRows = kGenWaves * kGenRows;

@@ -269,21 +269,22 @@ def test_staged_kernel_every_head_dim_pair(dtype, d):
 
 
 @pytest.mark.parametrize("T", [40, 200], ids=["eight_waves", "four_waves"])
-@pytest.mark.parametrize("S", [767, 768, 1500])
+@pytest.mark.parametrize("S,d_v", [(767, 128), (1500, 128), (1500, 16), (300, 256), (1500, 256)])
 @pytest.mark.parametrize("causal", [True, False], ids=["causal", "full"])
-def test_fp32_head_dim_128_with_and_without_the_next_keys_ahead(causal, S, T):
-    """fp32 at d = 128 loads the next keys ahead from 768 keys on; 72 and 312 tiles of 16 rows, on either
-    side of the device's CUs, take the key-split kernel's two shapes."""
+def test_fp32_head_dim_128_with_and_without_the_next_keys_ahead(causal, S, d_v, T):
+    """fp32 at d = 128 loads the next keys ahead beside d_v = 256 and not else; 72 and 312 tiles of 16
+    rows, on either side of the device's CUs, take the key-split kernel's two shapes (d_v = 256 has
+    one)."""
     from kernels import _lib
     assert (-(-T // 16) * 24 <= _lib.launch_plan()["num_cus"]) == (T == 40)
     g = torch.Generator().manual_seed(S + T)
     q = rand((2, 12, T, 128), g, torch.float32)
-    k, v = rand((2, 2, S, 128), g, torch.float32), rand((2, 2, S, 128), g, torch.float32)
-    lens = [S, S - 333]
+    k, v = rand((2, 2, S, 128), g, torch.float32), rand((2, 2, S, d_v), g, torch.float32)
+    lens = [S, S - 233]
     for b, n in enumerate(lens):
         k[b, :, n:] = PAD_VALUE
         v[b, :, n:] = PAD_VALUE
-    announce(f"[gpu] general fp32 d=128: T={T} S={S} causal={causal}")
+    announce(f"[gpu] general fp32 d=128 d_v={d_v}: T={T} S={S} causal={causal}")
     out = FlashAttention2Function.apply(q.to(DEV), k.to(DEV), v.to(DEV), causal,
                                         torch.tensor(lens, dtype=torch.int32, device=DEV))
     torch.cuda.synchronize()
