@@ -360,9 +360,12 @@ __global__ __launch_bounds__(64 * kGenWaves) void fa2_general_kernel(FwdParams p
 // merged through LDS at the end.  W = 4, or 8 (twice the key split) when the grid leaves a whole CU
 // to each work-group (d_v <= 128).  Bound by the latency of a pair's loads and, where two
 // work-groups share a CU, by the longer one's chain: wide V loads and pairing long with short tiles
-// took 1 x 12 x 512 x 128 fp32 from 36.0 to 25.9 us, 1 x 12 x 1000 x 256 bf16 from 142 to 87.
+// took 1 x 12 x 512 x 128 fp32 from 36.0 to 25.9 us, 1 x 12 x 1000 x 256 bf16 from 142 to 87; with the
+// next pair's keys ahead and the occupancy below they are at 24.0 and 66.
+
 // Two waves per SIMD, so that two work-groups of four share a CU, where their registers allow without
-// spilling.
+// spilling: left to itself the compiler takes more than 256 at d_v = 256 and in fp32 at d = 128 and 256
+// (fp32 32 / 256, 16 x 512 383 -> 229 us; 256 / 128, 4 x 1000 387 -> 324).
 template <class E, int D, int DV>
 constexpr int kSplitOcc =
     DV == 256 && (D == 256 || (D >= 64 && sizeof(typename Gen<E>::T) == 4)) ? 1 : 2;

@@ -40,8 +40,8 @@ inline GeneralKernel general_kernel(const GeneralCall& c) {
   // Fewer query rows than a work-group holds, or fewer work-groups than the device's CUs (256 on
   // MI355X): split each 16-row tile's keys over 4 waves instead (4x the work-groups, a quarter of
   // the chain).  fp32 always: its MFMAs are slow enough to cover the split kernel's loads, and
-  // staging bought nothing (1 x 12 x 1500 x 128 causal: staged 216 us, split 147; 4 x 1500 x 64:
-  // 247 and 218; 4096 x 128: 1,039 and 801).
+  // staging bought nothing (1 x 12 x 1500 x 128 causal: staged 217 us, split 130; 4 x 1500 x 64:
+  // 246 and 197; 4096 x 128: 1,040 and 669).
   const bool split = !c.bits16 || c.seqlen_q < kWgRows || tiles < c.n_cus;
   // The sizes of fa2_prefill_dims.hip.  12 heads, causal, us:
   //  * instead of the split kernel (d <= 64; at d = 256 it is the closer one to 64 bits), where its

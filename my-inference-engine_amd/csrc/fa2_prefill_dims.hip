@@ -17,9 +17,11 @@
 //   * The work-groups' order is that of the head-dim-128 kernel: heads sharing a kv head on one XCD,
 //     longest tiles first.
 // Measured (bf16, causal, 12 heads over 2 kv heads, before on the general kernels -> here; 4 x 2
-// unless said): 4 x 1000 x 64 36.6 -> 20.9 us, 1 x 1000 x 64 19.2 -> 18.0, 2 x 4 13.5;
-// 4 x 1500 x 64 66.9 -> 31.3, 2 x 4 53; 4 x 1200 x 32 34.2 -> 17.2; 2 x 1000 x 256 112.9 -> 56;
-// 1 x 4096 x 256 585 -> 170 (606 TFLOP/s).
+// unless said): 4 x 1000 x 64 37.7 -> 21.0 us, 1 x 1000 x 64 25.0 -> 2 x 4 13.7; 4 x 1500 x 64 67.7 ->
+// 32.0, 2 x 4 53; 4 x 1200 x 32 36.3 -> 19.8; 2 x 1000 x 256 112.6 -> 55.9; 1 x 4096 x 256 586 -> 200
+// (516 TFLOP/s, ten calls back to back).  The branch for large scores costs 0-2% of that at d = 64, 0-3%
+// at 32, 3-4% at 256 (the exponentials of two runs of keys are no longer scheduled across it; walking the
+// tile twice instead, or scaling the scores first, cost 2-3% at every size, and up to 20%).
 #include "fa2_common.h"
 #include "fa2_tiles.h"
 
@@ -200,7 +202,7 @@ __global__ __launch_bounds__(
   const auto exps = [&](const f32x16& s, u32x4 (&pb)[2]) {
     const float m_use = m_run == -INFINITY ? 0.f : m_run;
     float lt = 0.f;
-    if (exact) {
+    if (D > 64 ? exact : __builtin_expect(exact, false)) {
 #pragma clang fp contract(off)
 #pragma unroll
       for (int i = 0; i < 8; ++i) {
