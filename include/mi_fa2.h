@@ -31,7 +31,8 @@
  *   - Launches are asynchronous on `stream` (a hipStream_t); nothing is synchronised and nothing
  *     is allocated.  Entry points that need scratch take a caller-owned workspace whose size the
  *     matching *_workspace_size() returns; its contents need no initialisation.  Calls that
- *     overlap in time (other streams) must not share one workspace.
+ *     overlap in time (other streams; other threads on one stream, as a call may be two launches)
+ *     must not share one workspace.
  *   - Return value: MI_FA2_OK (0) or an error code; mi_fa2_last_error() then describes it.
  */
 #ifndef MI_FA2_H
@@ -116,7 +117,8 @@ MI_FA2_API int mi_fa2_set_clock_probe(uint64_t* probe);
  * seqlen_q == 1 runs the split-KV decode kernel, which needs the workspace; seqlen_q > 1 runs the
  * MFMA prefill kernel, which needs none.  Where few queries meet many keys, a non-zero size is
  * reported for seqlen_q > 1 too: with that workspace (16-byte aligned) the keys are split over
- * work-groups, without it the call runs unsplit.
+ * work-groups, without it the call runs unsplit, which is faster where the rows are far shorter
+ * than seqlen_k (the pieces follow seqlen_k).
  */
 MI_FA2_API size_t mi_fa2_fwd_workspace_size(int32_t batch, int32_t heads_q, int32_t heads_kv,
                                  int32_t seqlen_q, int32_t seqlen_k, int32_t head_dim);
